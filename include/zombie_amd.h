@@ -338,8 +338,9 @@ typedef struct zg_solve_options {
     int32_t regroup_interval; /* iterations between wavefront ballots that refill idle lanes */
     int32_t step_interval;    /* iterations (one BVH node visit each) between walk steps   */
     int32_t waves_per_cu;     /* persistent grid size = CUs * waves_per_cu (0 = auto)    */
-    int32_t count_visits;     /* 1: instrumented kernel counting the BVH node/primitive visits
-                                 of its own queries; 2: instead, at every query point, those of
+    int32_t count_visits;     /* 1: instrumented kernel counting the node/primitive visits of its
+                                 queries over the BVH's axis-aligned boxes (uninstrumented exact
+                                 queries read the oriented ones); 2: instead, at every query point, those of
                                  an exact nearest-first traversal from the root (the query's
                                  algorithmic work; walk on spheres only)                   */
     float distance_tolerance; /* tau in [0, 0.5): 0 = exact closest-point radii.  tau > 0 lets

@@ -76,6 +76,7 @@ struct DeviceBoundary {
     float* silNodes = nullptr;
     float* silCones = nullptr;
     float silConePrecision = 0.0f;
+    float4* obb = nullptr;       // oriented child boxes (absorbing)
     float* robinMax = nullptr;   // largest Robin coefficient per packed primitive
     BuiltBoundary host;  // sizes only after upload (vectors cleared; reflecting primIds kept)
     int64_t bytes = 0;
@@ -111,6 +112,7 @@ void freeBoundary(DeviceBoundary& b) {
     if (b.sil) (void)hipFree(b.sil);
     if (b.silNodes) (void)hipFree(b.silNodes);
     if (b.silCones) (void)hipFree(b.silCones);
+    if (b.obb) (void)hipFree(b.obb);
     if (b.robinMax) (void)hipFree(b.robinMax);
     b = DeviceBoundary();
 }
@@ -126,6 +128,49 @@ zg_status uploadBoundary(DeviceBoundary& d, BoundaryView& v) {
     v.nodes = d.nodes; v.prims = d.prims; v.primIds = d.primIds; v.sil = d.sil; v.silNodes = d.silNodes;
     v.silCones = d.silCones; v.silConePrecision = d.silConePrecision;
     v.nNodes = d.host.nNodes; v.nPrims = d.host.nPrims; v.nSil = d.host.nSil; v.nSilNodes = d.host.nSilNodes;
+    return ZG_OK;
+}
+
+// Adds the oriented child boxes to an uploaded boundary.  Without memory for them the boundary stays as
+// it is and exact queries use the axis-aligned boxes.
+template <int DIM, int W>
+zg_status buildObb(DeviceBoundary& d, BoundaryView& v) {
+    using L = NodeLayout<DIM, W>;
+    const int n = d.host.nNodes;
+    if (n == 0) return ZG_OK;
+    // primitives of every subtree: contiguous, since they are packed in leaf order; children come after
+    // their parent
+    std::vector<int2> ranges((size_t)n * W, make_int2(0, 0)), own(n);
+    for (int i = n - 1; i >= 0; i--) {
+        const float* nd = &d.host.nodes[(size_t)i * L::kFloats];
+        const int32_t* ch = reinterpret_cast<const int32_t*>(nd + L::kChildOffset);
+        int lo = INT32_MAX, hi = 0;
+        for (int k = 0; k < W; k++) {
+            if (ch[k] == 0) continue;   // empty slot: no child is the root
+            const int2 r = ch[k] < 0 ? make_int2(leafFirst(ch[k]), leafCount(ch[k])) : own[ch[k]];
+            ranges[(size_t)i * W + k] = r;
+            lo = std::min(lo, r.x); hi = std::max(hi, r.x + r.y);
+        }
+        own[i] = make_int2(lo, hi - lo);
+    }
+    const size_t bytes = (size_t)n * W * ObbLayout<DIM>::kVec * sizeof(float4);
+    float4* obb = nullptr;
+    int2* dr = nullptr;
+    hipError_t e = hipMalloc((void**)&obb, bytes);
+    if (e == hipSuccess) e = hipMalloc((void**)&dr, ranges.size() * sizeof(int2));
+    const bool noRoom = e == hipErrorOutOfMemory;
+    if (noRoom) (void)hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpy(dr, ranges.data(), ranges.size() * sizeof(int2), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = launchBuildObb(d.nodes, d.prims, DIM, W, n, dr, obb, 0);
+    if (e == hipSuccess) e = hipStreamSynchronize(0);
+    if (dr) (void)hipFree(dr);
+    if (e != hipSuccess) {
+        if (obb) (void)hipFree(obb);
+        return noRoom ? ZG_OK : fail(ZG_ERR_DEVICE, "oriented boxes: %s", hipGetErrorString(e));
+    }
+    d.obb = obb;
+    v.obb = obb;
+    d.bytes += (int64_t)bytes;
     return ZG_OK;
 }
 
@@ -260,6 +305,9 @@ zg_status zg_scene_create(int32_t dim, const float* V, int64_t nV, const int32_t
         return fail(ZG_ERR_INVALID_ARGUMENT, "scene build failed: %s", e.what());
     }
     zg_status st = uploadBoundary(s->abs, s->view.abs);
+    if (st == ZG_OK)
+        st = dim == 2 ? (o.bvh_width == 4 ? buildObb<2, 4>(s->abs, s->view.abs) : buildObb<2, 8>(s->abs, s->view.abs))
+                      : (o.bvh_width == 4 ? buildObb<3, 4>(s->abs, s->view.abs) : buildObb<3, 8>(s->abs, s->view.abs));
     if (st == ZG_OK) st = uploadBoundary(s->refl, s->view.refl);
     if (st != ZG_OK) { freeBoundary(s->abs); freeBoundary(s->refl); delete s; return st; }
     s->view.dim = dim; s->view.width = o.bvh_width;
@@ -476,6 +524,7 @@ zg_status zg_sample_reflecting(const zg_scene* s, int64_t n, const float* x, con
 // A batch of instances walked by one persistent launch (the scenes stay owned by the caller).
 struct zg_batch {
     int n = 0, dim = 3, width = 8, device = 0, maxDepth = 0;
+    bool hasObb = true;   // every instance has oriented boxes
     std::vector<const zg_scene*> scenes;
     std::vector<zg_pde> pdes;
     InstanceDesc* table = nullptr;
@@ -598,6 +647,7 @@ zg_status prepareSolve(const zg_scene* s, const zg_batch* b, const zg_pde* pde, 
     P.seed = o.seed; P.streamOffset = o.stream_offset;
     P.countMode = o.count_visits;
     P.relax2 = (1.0f - o.distance_tolerance) * (1.0f - o.distance_tolerance);
+    P.exact = o.distance_tolerance == 0.0f && o.count_visits == 0 && (s ? s->view.abs.obb != nullptr : b->hasObb);
     float e2 = 2.0f * ws->epsilon_shell_for_absorbing_boundary;
     P.guard2 = e2 * e2 / P.relax2;
 
@@ -962,9 +1012,10 @@ zg_status zg_batch_create(int32_t nInstances, const zg_scene* const* scenes, con
         zg_status st = checkPde(&pdes[i], 3);
         if (st != ZG_OK) { delete b; return st; }
         b->width = s->width; b->device = s->device; b->maxDepth = std::max(b->maxDepth, s->info.absorbing_depth);
+        b->hasObb = b->hasObb && s->view.abs.obb;
         InstanceDesc& d = host[i];
         std::memset(&d, 0, sizeof(d));
-        d.nodes = s->view.abs.nodes; d.prims = s->view.abs.prims; d.nNodes = s->view.abs.nNodes; d.nPrims = s->view.abs.nPrims;
+        d.nodes = s->view.abs.nodes; d.prims = s->view.abs.prims; d.obb = s->view.abs.obb; d.nNodes = s->view.abs.nNodes; d.nPrims = s->view.abs.nPrims;
         for (int a = 0; a < 3; a++) { d.dmin[a] = s->view.dmin[a]; d.dmax[a] = s->view.dmax[a]; }
         d.pde = pdes[i];
         b->scenes.push_back(s);

@@ -23,6 +23,7 @@ enum CounterSlot {
 struct InstanceDesc {
     const float* nodes;
     const float* prims;
+    const float4* obb;
     int32_t nNodes;
     int32_t nPrims;
     float dmin[3], dmax[3];
@@ -54,6 +55,7 @@ struct WosParams {
     float relax2;        // (1 - distance_tolerance)^2
     float guard2;        // relaxation only when best^2 > guard2 (keeps the shell test exact)
     int32_t nInstances;  // batched solves: size of the instance table
+    int32_t exact;       // distance tolerance 0 and oriented boxes present: queries over the oriented boxes
     int32_t countMode;   // COUNT kernels: 1 = visits of the kernel's own queries, 2 = visits of an exact
                          // nearest-first traversal from the root at every query point
     double* accSum;
@@ -134,6 +136,10 @@ struct MergeParams {
     double* gDeriv;
 };
 
+// oriented child boxes of a boundary's BVH (layout.h); ranges[node * W + slot] = first packed primitive and
+// number of primitives of that child's subtree (0: empty slot)
+hipError_t launchBuildObb(const float* nodes, const float* prims, int dim, int width, int nNodes, const int2* ranges,
+                          float4* obb, hipStream_t s);
 hipError_t launchFillZero(uint64_t* p, int64_t nWords, hipStream_t s);
 // solves without a report: their error flags are latched on the device and reported by zg_synchronize
 hipError_t launchLatchErrors(const unsigned long long* counters, hipStream_t s);

@@ -13,6 +13,8 @@
 //   2D segment  :  4 floats  a.xy b.xy                                          (16 B)
 //                 + int32 caller index in a separate array
 #pragma once
+#include <hip/hip_runtime.h>
+
 #include <cstdint>
 
 namespace zg {
@@ -27,6 +29,16 @@ struct NodeLayout {
     static constexpr int kFloats = ((kRawFloats + 15) / 16) * 16;
     static constexpr int kBytes = kFloats * 4;
     static constexpr int kChildOffset = kBoxFloats;
+};
+
+// Oriented boxes of the same tree (same node indices, child slots and child codes), read by exact
+// closest-point queries: node n holds its W children one after the other,
+//   3D  64 B: centre.xyz, code; axis0.xyz, half0; axis1.xyz, half1; axis2.xyz, half2
+//   2D  32 B: centre.xy, axis0.xy; half0, half1 (axis1 = axis0 turned by 90 degrees), code, 0
+// An empty slot has half extents of -kEmptyBox: its distance overflows to +inf.
+template <int DIM>
+struct ObbLayout {
+    static constexpr int kVec = DIM == 3 ? 4 : 2;   // float4 per child
 };
 
 template <int DIM>
@@ -54,6 +66,7 @@ struct BoundaryView {
                            // 3D: axis.xyz, sin; cos, 0, 0, 0)
     float silConePrecision;// the silhouette precision the cones' margin covers
     const float* robinMax; // 2D reflecting: largest Robin coefficient per packed primitive (null: 0)
+    const float4* obb;     // absorbing: nNodes * W oriented child boxes (null: queries use the nodes' boxes)
     int32_t nNodes;
     int32_t nPrims;
     int32_t nSil;

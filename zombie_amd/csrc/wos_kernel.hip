@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
+#include <type_traits>
 
 #include "device.h"
 #include "kernels.h"
@@ -104,6 +105,7 @@ __global__ void __launch_bounds__(256) rayKernel(BoundaryView b, int64_t n, cons
 struct WalkView {
     const float* nodes;
     const float* prims;
+    const float4* obb;
     int nNodes;
 };
 
@@ -164,7 +166,8 @@ ZG_DEV Vec<D> cvField(const WosParams& P, const Vec<D>& x) {
 // random numbers of the first (the reference replays its saved generator).  The walk then goes
 // on from the boundary point as a plain walk; its estimate feeds the solution statistics and the
 // gradient estimate (boundary term - cv) * grad P / P + (first source - cv) * grad G / (pdf |G|).
-template <int D, int W, bool COUNT, bool BATCH, bool SCREENED, bool SPLIT = false, bool GRAD = false>
+// EXACT = true (distance tolerance 0, no visit counting): queries over the oriented boxes.
+template <int D, int W, bool COUNT, bool BATCH, bool SCREENED, bool EXACT, bool SPLIT = false, bool GRAD = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WosOccupancy<W>::kWaves, 8)))
 wosKernel(WosParams P) {
     unsigned long long spill[kSpillStack];
@@ -176,7 +179,7 @@ wosKernel(WosParams P) {
     const uint32_t streamOffset = P.streamOffsetDev ? *P.streamOffsetDev : P.streamOffset;
     // scene / PDE of the current walk: uniform, or the lane's instance in batched solves
     const InstanceDesc* inst = nullptr;
-    WalkView view{P.scene.abs.nodes, P.scene.abs.prims, P.scene.abs.nNodes};
+    WalkView view{P.scene.abs.nodes, P.scene.abs.prims, P.scene.abs.obb, P.scene.abs.nNodes};
     float sigma = P.pde.absorption_coeff;
     // the PDE comes from the kernel arguments: walks here are cheap enough per step that reading
     // it from device memory at every use (as the walk-on-stars kernel does) cost 3.7x on 2D scenes
@@ -203,7 +206,7 @@ wosKernel(WosParams P) {
     // gradient walks: boundary / source gradient directions, first-step source term, control variates
     Vec<D> gB = vzero<D>(), gS = vzero<D>();
     float fsc = 0.0f, cvB = 0.0f, cvS = 0.0f;
-    ClosestQuery<D> q;
+    std::conditional_t<EXACT, ExactQuery<D>, ClosestQuery<D>> q;
     q.begin(FLT_MAX, 1.0f, 0.0f);
     // block counters in LDS: walks per completion code, steps, walks started
     __shared__ unsigned long long blk[6];
@@ -361,6 +364,7 @@ wosKernel(WosParams P) {
         if (BATCH) {
             inst = P.instances + P.instanceOf[p];
             view.nodes = inst->nodes; view.prims = inst->prims; view.nNodes = inst->nNodes;
+            view.obb = inst->obb;
             sigma = inst->pde.absorption_coeff;
             ball.sqrtLambda = __builtin_sqrtf(sigma);
         }
@@ -780,10 +784,15 @@ hipError_t launchRay(const SceneView& sv, int boundary, int64_t n, const float* 
     return hipGetLastError();
 }
 
+// the walk kernel of a solve: EXACT where the host found oriented boxes and a zero tolerance
 hipError_t launchWos(const WosParams& P, int dim, int width, bool count, bool screened, bool split, int gridBlocks,
                      hipStream_t s) {
     dim3 g(gridBlocks), bl(256);
-#define ZG_WOS(D, Wd, C, S, SP) hipLaunchKernelGGL((wosKernel<D, Wd, C, false, S, SP>), g, bl, kStackLdsBytes, s, P)
+#define ZG_WOS(D, Wd, C, S, SP)                                                                                        \
+    do {                                                                                                               \
+        if (P.exact && !C) hipLaunchKernelGGL((wosKernel<D, Wd, false, false, S, true, SP>), g, bl, kStackLdsBytes, s, P);  \
+        else hipLaunchKernelGGL((wosKernel<D, Wd, C, false, S, false, SP>), g, bl, kStackLdsBytes, s, P);              \
+    } while (0)
     if (split) {   // no visit counting with splitting
         if (dim == 2) { if (width == 4) ZG_WOS(2, 4, false, false, true); else ZG_WOS(2, 8, false, false, true); }
         else if (screened) { if (width == 4) ZG_WOS(3, 4, false, true, true); else ZG_WOS(3, 8, false, true, true); }
@@ -805,7 +814,11 @@ hipError_t launchWos(const WosParams& P, int dim, int width, bool count, bool sc
 hipError_t launchWosBatch(const WosParams& P, int width, bool count, bool screened, bool split, int gridBlocks,
                           hipStream_t s) {
     dim3 g(gridBlocks), bl(256);
-#define ZG_WOSB(Wd, C, S, SP) hipLaunchKernelGGL((wosKernel<3, Wd, C, true, S, SP>), g, bl, kStackLdsBytes, s, P)
+#define ZG_WOSB(Wd, C, S, SP)                                                                                          \
+    do {                                                                                                               \
+        if (P.exact && !C) hipLaunchKernelGGL((wosKernel<3, Wd, false, true, S, true, SP>), g, bl, kStackLdsBytes, s, P);   \
+        else hipLaunchKernelGGL((wosKernel<3, Wd, C, true, S, false, SP>), g, bl, kStackLdsBytes, s, P);               \
+    } while (0)
     if (split) {
         if (screened) { if (width == 4) ZG_WOSB(4, false, true, true); else ZG_WOSB(8, false, true, true); }
         else { if (width == 4) ZG_WOSB(4, false, false, true); else ZG_WOSB(8, false, false, true); }
@@ -823,7 +836,11 @@ hipError_t launchWosBatch(const WosParams& P, int width, bool count, bool screen
 hipError_t launchWosGrad(const WosParams& P, int dim, int width, bool screened, bool split, int gridBlocks,
                          hipStream_t s) {
     dim3 g(gridBlocks), bl(256);
-#define ZG_WOSG(D, Wd, S, SP) hipLaunchKernelGGL((wosKernel<D, Wd, false, false, S, SP, true>), g, bl, kStackLdsBytes, s, P)
+#define ZG_WOSG(D, Wd, S, SP)                                                                                          \
+    do {                                                                                                               \
+        if (P.exact) hipLaunchKernelGGL((wosKernel<D, Wd, false, false, S, true, SP, true>), g, bl, kStackLdsBytes, s, P);  \
+        else hipLaunchKernelGGL((wosKernel<D, Wd, false, false, S, false, SP, true>), g, bl, kStackLdsBytes, s, P);    \
+    } while (0)
     if (dim == 2) {
         if (split) { if (width == 4) ZG_WOSG(2, 4, false, true); else ZG_WOSG(2, 8, false, true); }
         else { if (width == 4) ZG_WOSG(2, 4, false, false); else ZG_WOSG(2, 8, false, false); }
