@@ -77,6 +77,7 @@ struct DeviceBoundary {
     float* silCones = nullptr;
     float silConePrecision = 0.0f;
     float4* obb = nullptr;       // oriented child boxes (absorbing)
+    float2* primEntry = nullptr; // entry record per packed primitive (absorbing)
     float* robinMax = nullptr;   // largest Robin coefficient per packed primitive
     BuiltBoundary host;  // sizes only after upload (vectors cleared; reflecting primIds kept)
     int64_t bytes = 0;
@@ -113,6 +114,7 @@ void freeBoundary(DeviceBoundary& b) {
     if (b.silNodes) (void)hipFree(b.silNodes);
     if (b.silCones) (void)hipFree(b.silCones);
     if (b.obb) (void)hipFree(b.obb);
+    if (b.primEntry) (void)hipFree(b.primEntry);
     if (b.robinMax) (void)hipFree(b.robinMax);
     b = DeviceBoundary();
 }
@@ -131,7 +133,7 @@ zg_status uploadBoundary(DeviceBoundary& d, BoundaryView& v) {
     return ZG_OK;
 }
 
-// Adds the oriented child boxes to an uploaded boundary.  Without memory for them the boundary stays as
+// Adds the oriented child boxes and the entry nodes to an uploaded boundary.  Without memory for them the boundary stays as
 // it is and exact queries use the axis-aligned boxes.
 template <int DIM, int W>
 zg_status buildObb(DeviceBoundary& d, BoundaryView& v) {
@@ -141,36 +143,48 @@ zg_status buildObb(DeviceBoundary& d, BoundaryView& v) {
     // primitives of every subtree: contiguous, since they are packed in leaf order; children come after
     // their parent
     std::vector<int2> ranges((size_t)n * W, make_int2(0, 0)), own(n);
+    std::vector<int32_t> leafSlots;
     for (int i = n - 1; i >= 0; i--) {
         const float* nd = &d.host.nodes[(size_t)i * L::kFloats];
         const int32_t* ch = reinterpret_cast<const int32_t*>(nd + L::kChildOffset);
         int lo = INT32_MAX, hi = 0;
         for (int k = 0; k < W; k++) {
             if (ch[k] == 0) continue;   // empty slot: no child is the root
+            if (ch[k] < 0) leafSlots.push_back(i * W + k);
             const int2 r = ch[k] < 0 ? make_int2(leafFirst(ch[k]), leafCount(ch[k])) : own[ch[k]];
             ranges[(size_t)i * W + k] = r;
             lo = std::min(lo, r.x); hi = std::max(hi, r.x + r.y);
         }
         own[i] = make_int2(lo, hi - lo);
     }
-    const size_t bytes = (size_t)n * W * ObbLayout<DIM>::kVec * sizeof(float4);
+    const size_t all = (size_t)n + leafSlots.size() * kEntryLevels;
+    if (all > (size_t)INT32_MAX / W) return ZG_OK;
+    const size_t bytes = all * W * ObbLayout<DIM>::kVec * sizeof(float4);
     float4* obb = nullptr;
+    float2* primEntry = nullptr;
     int2* dr = nullptr;
+    int32_t* dl = nullptr;
     hipError_t e = hipMalloc((void**)&obb, bytes);
+    if (e == hipSuccess) e = hipMalloc((void**)&primEntry, (size_t)d.host.nPrims * sizeof(float2));
     if (e == hipSuccess) e = hipMalloc((void**)&dr, ranges.size() * sizeof(int2));
+    if (e == hipSuccess) e = hipMalloc((void**)&dl, leafSlots.size() * sizeof(int32_t));
     const bool noRoom = e == hipErrorOutOfMemory;
     if (noRoom) (void)hipGetLastError();
     if (e == hipSuccess) e = hipMemcpy(dr, ranges.data(), ranges.size() * sizeof(int2), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(dl, leafSlots.data(), leafSlots.size() * sizeof(int32_t), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = launchBuildObb(d.nodes, d.prims, DIM, W, n, dr, obb, 0);
+    if (e == hipSuccess) e = launchBuildEntries(d.nodes, DIM, W, n, dl, (int)leafSlots.size(), obb, primEntry, 0);
     if (e == hipSuccess) e = hipStreamSynchronize(0);
     if (dr) (void)hipFree(dr);
+    if (dl) (void)hipFree(dl);
     if (e != hipSuccess) {
         if (obb) (void)hipFree(obb);
+        if (primEntry) (void)hipFree(primEntry);
         return noRoom ? ZG_OK : fail(ZG_ERR_DEVICE, "oriented boxes: %s", hipGetErrorString(e));
     }
-    d.obb = obb;
-    v.obb = obb;
-    d.bytes += (int64_t)bytes;
+    d.obb = obb; d.primEntry = primEntry;
+    v.obb = obb; v.primEntry = primEntry;
+    d.bytes += (int64_t)(bytes + (size_t)d.host.nPrims * sizeof(float2));
     return ZG_OK;
 }
 
@@ -1015,7 +1029,7 @@ zg_status zg_batch_create(int32_t nInstances, const zg_scene* const* scenes, con
         b->hasObb = b->hasObb && s->view.abs.obb;
         InstanceDesc& d = host[i];
         std::memset(&d, 0, sizeof(d));
-        d.nodes = s->view.abs.nodes; d.prims = s->view.abs.prims; d.obb = s->view.abs.obb; d.nNodes = s->view.abs.nNodes; d.nPrims = s->view.abs.nPrims;
+        d.nodes = s->view.abs.nodes; d.prims = s->view.abs.prims; d.obb = s->view.abs.obb; d.primEntry = s->view.abs.primEntry; d.nNodes = s->view.abs.nNodes; d.nPrims = s->view.abs.nPrims;
         for (int a = 0; a < 3; a++) { d.dmin[a] = s->view.dmin[a]; d.dmax[a] = s->view.dmax[a]; }
         d.pde = pdes[i];
         b->scenes.push_back(s);

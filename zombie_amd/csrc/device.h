@@ -921,6 +921,20 @@ ZG_DEV void childBounds(const float4* obb, int idx, const Vec<D>& x, float (&d2)
     }
 }
 
+// node where an exact query starts whose seed (packed primitive prim) lies at squared distance s2: the
+// smallest entry of the seed's leaf that reaches 2 s, the root beyond the last one
+ZG_DEV int entryNode(const float2* primEntry, int prim, float s2) {
+    const float2 e = primEntry[prim];
+    int level = 0;
+    float r2 = e.x;
+#pragma unroll
+    for (int j = 0; j < kEntryLevels; j++) {
+        level += s2 > r2 ? 1 : 0;
+        r2 *= kEntryRatio * kEntryRatio;
+    }
+    return level < kEntryLevels ? __float_as_int(e.y) + level : 0;
+}
+
 // Exact form of ClosestQuery over the oriented boxes (same work items, order and restart rule).
 //
 // A triangle's axis-aligned box reaches about an edge length towards the query point, so a query far from a

@@ -24,6 +24,7 @@ struct InstanceDesc {
     const float* nodes;
     const float* prims;
     const float4* obb;
+    const float2* primEntry;
     int32_t nNodes;
     int32_t nPrims;
     float dmin[3], dmax[3];
@@ -140,6 +141,9 @@ struct MergeParams {
 // number of primitives of that child's subtree (0: empty slot)
 hipError_t launchBuildObb(const float* nodes, const float* prims, int dim, int width, int nNodes, const int2* ranges,
                           float4* obb, hipStream_t s);
+// entry nodes (layout.h), after the nNodes * width boxes of obb; leafSlots[i] = node * width + slot of leaf i
+hipError_t launchBuildEntries(const float* nodes, int dim, int width, int nNodes, const int32_t* leafSlots, int nLeaves,
+                              float4* obb, float2* primEntry, hipStream_t s);
 hipError_t launchFillZero(uint64_t* p, int64_t nWords, hipStream_t s);
 // solves without a report: their error flags are latched on the device and reported by zg_synchronize
 hipError_t launchLatchErrors(const unsigned long long* counters, hipStream_t s);

@@ -41,6 +41,22 @@ struct ObbLayout {
     static constexpr int kVec = DIM == 3 ? 4 : 2;   // float4 per child
 };
 
+// Entry nodes.  An exact query of a walk knows a primitive close to its point x: the closest one of the query
+// before (the seed), at distance s.  Whatever is closest to x lies within s of x, hence within 2 s of the
+// seed.  For every leaf, kEntryLevels more nodes of oriented boxes after the BVH's own (indices nNodes +
+// leaf * kEntryLevels + level) hold a cover, in at most W items, of everything within reach_level =
+// kEntryReach * diagonal of the leaf's box * kEntryRatio^level of that box; the query starts at the smallest
+// level with 2 s <= reach_level instead of at the root.  primEntry holds, for every packed primitive,
+// (reach_0 / 2)^2 and (int bits) the level-0 entry of its leaf.
+//
+// Node visits per query on the 81,920-triangle sphere 12.7 -> 8.8, 100,000 points x 64 walks 66.0 -> 58.5 ms;
+// 12 screened instances 61.3 -> 58.0 ms, 1,024 segments in 2D 13.5 -> 13.1 ms.  Levels x reach x ratio of
+// 4 x 0.25 x 4 / 3 x 0.25 x 4 / 2 x 0.5 x 8 / 4 x 0.1 x 4 ran 57.9 / 57.4 / 58.5 / 57.1 ms there: two
+// levels need half of four's memory (W * 64 B a level and leaf in 3D) for 1-2%.
+constexpr int kEntryLevels = 2;
+constexpr float kEntryReach = 0.5f;
+constexpr float kEntryRatio = 8.0f;
+
 template <int DIM>
 struct PrimLayout {
     static constexpr int kFloats = DIM == 3 ? 12 : 4;
@@ -66,7 +82,9 @@ struct BoundaryView {
                            // 3D: axis.xyz, sin; cos, 0, 0, 0)
     float silConePrecision;// the silhouette precision the cones' margin covers
     const float* robinMax; // 2D reflecting: largest Robin coefficient per packed primitive (null: 0)
-    const float4* obb;     // absorbing: nNodes * W oriented child boxes (null: queries use the nodes' boxes)
+    const float4* obb;     // absorbing: nNodes * W oriented child boxes, then the entry nodes (null: queries
+                           // use the nodes' boxes)
+    const float2* primEntry;  // absorbing, with obb: entry record per packed primitive
     int32_t nNodes;
     int32_t nPrims;
     int32_t nSil;

@@ -149,4 +149,94 @@ hipError_t launchBuildObb(const float* nodes, const float* prims, int dim, int w
     return hipGetLastError();
 }
 
+// One thread builds one entry node: the cover starts as the root's children within reach, and its largest
+// inner item is replaced by that item's children within reach for as long as the result fits in W slots, so
+// that an entry sits as deep in the tree as W items allow.
+template <int D, int W>
+__global__ void __launch_bounds__(256) buildEntriesKernel(const float* __restrict__ nodes, int nNodes,
+                                                          const int32_t* __restrict__ leafSlots, int nLeaves,
+                                                          float4* __restrict__ obb, float2* __restrict__ primEntry) {
+    using L = NodeLayout<D, W>;
+    constexpr int V = ObbLayout<D>::kVec;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (int64_t)nLeaves * kEntryLevels) return;
+    const int leaf = (int)(t / kEntryLevels), level = (int)(t % kEntryLevels);
+    const float* ln = nodes + (size_t)(leafSlots[leaf] / W) * L::kFloats;
+    const int slot = leafSlots[leaf] % W;
+    float lo[D], hi[D], diag2 = 0.0f, mag = 0.0f;
+    for (int a = 0; a < D; a++) {
+        lo[a] = ln[a * W + slot];
+        hi[a] = ln[(D + a) * W + slot];
+        diag2 += (hi[a] - lo[a]) * (hi[a] - lo[a]);
+        mag = fmaxf(mag, fmaxf(fabsf(lo[a]), fabsf(hi[a])));
+    }
+    float reach = kEntryReach * __builtin_sqrtf(diag2);
+    if (level == 0) {
+        const int code = __float_as_int(ln[L::kChildOffset + slot]);
+        const int first = leafFirstD(code), cnt = leafCountD(code);
+        for (int i = first; i < first + cnt; i++)
+            primEntry[i] = make_float2(0.25f * reach * reach, __int_as_float(nNodes + leaf * kEntryLevels));
+    }
+    // the cover's radius: the reach plus what rounding can add to the distances that are compared with it
+    // (coordinates of magnitude mag leave a few ulps of mag in a computed distance)
+    for (int j = 0; j < level; j++) reach *= kEntryRatio;
+    reach = reach * 1.001f + 8e-6f * mag;
+    const float reach2 = reach * reach;
+
+    int src[W], code[W];   // child slot (node * W + k) an item comes from, and its code
+    float size[W];
+    bool open[W];          // an inner item that may still be replaced by its children
+    int n = 1;
+    src[0] = 0; code[0] = 0; open[0] = true; size[0] = FLT_MAX;   // the root: replaced at once
+    for (;;) {
+        int pick = -1;
+        for (int i = 0; i < n; i++)
+            if (open[i] && (pick < 0 || size[i] > size[pick])) pick = i;
+        if (pick < 0) break;
+        const int node = code[pick];
+        const float* nd = nodes + (size_t)node * L::kFloats;
+        int keep[W], m = 0;
+        for (int k = 0; k < W; k++) {
+            if (__float_as_int(nd[L::kChildOffset + k]) == 0) continue;   // empty slot
+            float d2 = 0.0f;
+            for (int a = 0; a < D; a++) {
+                const float g = fmaxf(fmaxf(nd[a * W + k] - hi[a], lo[a] - nd[(D + a) * W + k]), 0.0f);
+                d2 += g * g;
+            }
+            if (!(d2 > reach2)) keep[m++] = k;
+        }
+        if (n - 1 + m > W) { open[pick] = false; continue; }
+        n--;   // the picked item leaves, its children within reach enter
+        src[pick] = src[n]; code[pick] = code[n]; open[pick] = open[n]; size[pick] = size[n];
+        for (int q = 0; q < m; q++, n++) {
+            const int k = keep[q];
+            src[n] = node * W + k;
+            code[n] = __float_as_int(nd[L::kChildOffset + k]);
+            open[n] = !isLeaf(code[n]);
+            size[n] = 0.0f;
+            for (int a = 0; a < D; a++) size[n] += nd[(D + a) * W + k] - nd[a * W + k];
+        }
+    }
+    float4* out = obb + (size_t)(nNodes + (int64_t)leaf * kEntryLevels + level) * W * V;
+    for (int k = 0; k < W; k++)
+        for (int v = 0; v < V; v++) {
+            // an empty slot: half extents of -kEmptyBox
+            float4 e = D == 3 ? make_float4(0.0f, 0.0f, 0.0f, v ? -kEmptyBox : 0.0f)
+                              : (v ? make_float4(-kEmptyBox, -kEmptyBox, 0.0f, 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+            if (k < n) e = obb[(size_t)src[k] * V + v];
+            out[k * V + v] = e;
+        }
+}
+
+hipError_t launchBuildEntries(const float* nodes, int dim, int width, int nNodes, const int32_t* leafSlots, int nLeaves,
+                              float4* obb, float2* primEntry, hipStream_t s) {
+    if (nLeaves <= 0) return hipSuccess;
+    dim3 g((unsigned)(((int64_t)nLeaves * kEntryLevels + 255) / 256)), bl(256);
+    if (dim == 2 && width == 4) hipLaunchKernelGGL((buildEntriesKernel<2, 4>), g, bl, 0, s, nodes, nNodes, leafSlots, nLeaves, obb, primEntry);
+    else if (dim == 2) hipLaunchKernelGGL((buildEntriesKernel<2, 8>), g, bl, 0, s, nodes, nNodes, leafSlots, nLeaves, obb, primEntry);
+    else if (width == 4) hipLaunchKernelGGL((buildEntriesKernel<3, 4>), g, bl, 0, s, nodes, nNodes, leafSlots, nLeaves, obb, primEntry);
+    else hipLaunchKernelGGL((buildEntriesKernel<3, 8>), g, bl, 0, s, nodes, nNodes, leafSlots, nLeaves, obb, primEntry);
+    return hipGetLastError();
+}
+
 }  // namespace zg

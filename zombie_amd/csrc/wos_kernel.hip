@@ -492,7 +492,9 @@ wosKernel(WosParams P) {
             // distance seeds the bound, so the traversal from the root prunes early
             Prim<D> pr; pr.load(view.prims, ycPrim);
             Vec<D> qq;
-            q.seed(qq, ycPrim, pr.closest2(x, qq));
+            const float s2 = pr.closest2(x, qq);
+            q.seed(qq, ycPrim, s2);
+            if (EXACT) q.item = entryNode(BATCH ? inst->primEntry : P.scene.abs.primEntry, ycPrim, s2);
             if (COUNT) vc.prims++;
         }
     };
