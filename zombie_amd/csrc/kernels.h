@@ -178,7 +178,7 @@ hipError_t launchSdfInside(const zg_function& sdf, int dim, int64_t n, const flo
 // boundary value caching splat
 hipError_t launchBvcSplat(int dim, float absorption, const zg_bvc_samples& S, const zg_bvc_eval_points& E,
                           const zg_bvc_statistics& out, float radiusClamp, float kreg, float robinCutoff, float cutoffA,
-                          float cutoffR, hipStream_t s);
+                          float cutoffR, int targetWaves, hipStream_t s);
 // read-bandwidth probe
 hipError_t launchReadProbe(const void* buf, int64_t bytes, int reps, int blocks, float* sink, hipStream_t s);
 // walk on stars (2D)
