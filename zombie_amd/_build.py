@@ -29,7 +29,7 @@ HIP_FLAGS = [
     "-Wno-unused-result",
 ]
 
-SOURCES = ["bvh_build.cpp", "abi.cpp", "wos_kernel.hip", "wost_kernel.hip", "mlp_kernels.hip", "probe_kernel.hip",
+SOURCES = ["bvh_build.cpp", "abi.cpp", "wos_kernel.hip", "wost_kernel.hip", "mlp_kernels.hip", "mlp_fused.hip", "probe_kernel.hip",
            "bvc_kernel.hip", "obb_kernel.hip", "sdf_kernel.hip", "spatial_sort.cpp", "noalloc.hip"]
 
 

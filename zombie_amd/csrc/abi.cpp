@@ -1197,6 +1197,8 @@ zg_status zg_mlp_create(const zg_mlp_config* cfg, int64_t maxBatch, zg_mlp** out
     }
     d.nParams = off;
     d.maxRows = maxBatch;
+    const bool fused = mlpFusable(d.shape);
+    const int64_t rows = (maxBatch + 63) / 64 * 64;   // the fused layers work on whole tiles of 64 rows
     // host initialisation: PyTorch-style U(-1/sqrt(in), 1/sqrt(in)) weights and biases,
     // Gaussian frequencies
     std::mt19937_64 gen(cfg->seed);
@@ -1221,14 +1223,39 @@ zg_status zg_mlp_create(const zg_mlp_config* cfg, int64_t maxBatch, zg_mlp** out
     if (e == hipSuccess) e = mlpAlloc(m, &d.wBf, off);
     if (e == hipSuccess) e = mlpAlloc(m, &d.bfIndex, off);
     if (e == hipSuccess) e = mlpAlloc(m, &d.freq, (int64_t)freq.size());
-    if (e == hipSuccess) e = mlpAlloc(m, &d.phi, maxBatch * F2);
-    if (e == hipSuccess) e = mlpAlloc(m, &d.dphi, maxBatch * F2);
+    if (e == hipSuccess) e = mlpAlloc(m, &d.phi, rows * F2);
     for (int l = 0; l < L && e == hipSuccess; l++) {
-        e = mlpAlloc(m, &d.pre[l], maxBatch * H);
-        if (e == hipSuccess) e = mlpAlloc(m, &d.act[l], maxBatch * H);
+        // fused: the bf16 gradients of the pre-activations take the place of these
+        e = mlpAlloc(m, &d.pre[l], fused ? rows * H / 2 : maxBatch * H);
+        if (e == hipSuccess) e = mlpAlloc(m, &d.act[l], rows * H);
     }
-    if (e == hipSuccess) e = mlpAlloc(m, &d.dz[0], maxBatch * H);
-    if (e == hipSuccess) e = mlpAlloc(m, &d.dz[1], maxBatch * H);
+    if (fused) {
+        std::vector<int64_t> at, tr(off, -1);
+        auto place = [](int64_t k, int64_t n, int64_t K) {   // mlp.h, wBfT
+            return ((n / 16 * (K / 32) + k / 32) * 64 + k / 8 % 4 * 16 + n % 16) * 8 + k % 8;
+        };
+        for (int l = 0; l < L; l++) {
+            const int in = l == 0 ? F2 : H;
+            for (int64_t i = 0; i < (int64_t)in * H; i++) {
+                const int64_t p = d.wOffset[l] + i;
+                at.push_back(p);
+                bfIndex[p] = d.wOffset[l] + place(i % in, i / in, in);
+                tr[p] = d.wOffset[l] + place(i / in, i % in, H);
+            }
+        }
+        d.nHiddenWeights = (int64_t)at.size();
+        if (e == hipSuccess) e = mlpAlloc(m, &d.wBfT, off);
+        if (e == hipSuccess) e = mlpAlloc(m, &d.bfIndexT, off);
+        if (e == hipSuccess) e = mlpAlloc(m, &d.weightAt, d.nHiddenWeights);
+        if (e == hipSuccess) e = mlpAlloc(m, &d.part, (int64_t)kMlpSplits * (128 / H) * off);
+        if (e == hipSuccess) e = mlpAlloc(m, &d.partSmall, (int64_t)2 * kMlpFusedBlocks * ((L + 1) * H + 2));
+        if (e == hipSuccess) e = hipMemcpy(d.bfIndexT, tr.data(), off * 8, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(d.weightAt, at.data(), at.size() * 8, hipMemcpyHostToDevice);
+    } else {
+        if (e == hipSuccess) e = mlpAlloc(m, &d.dphi, maxBatch * F2);
+        if (e == hipSuccess) e = mlpAlloc(m, &d.dz[0], maxBatch * H);
+        if (e == hipSuccess) e = mlpAlloc(m, &d.dz[1], maxBatch * H);
+    }
     if (e == hipSuccess) e = mlpAlloc(m, &d.loss, 1);
     if (e == hipSuccess) e = hipMemcpy(d.theta, theta.data(), off * 4, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d.bfIndex, bfIndex.data(), off * 8, hipMemcpyHostToDevice);
@@ -1280,20 +1307,23 @@ zg_status zg_mlp_get_frequencies(const zg_mlp* m, float* host, int64_t count) {
     return ok();
 }
 
-static zg_status mlpGradientsImpl(zg_mlp* m, const float* x, const float* y, int64_t batch, hipStream_t s) {
+// gradients and loss, and the Adam step if lr is given
+static zg_status mlpGradientsImpl(zg_mlp* m, const float* x, const float* y, int64_t batch, const float* lr, hipStream_t s) {
     if (!m || !x || !y) return fail(ZG_ERR_INVALID_ARGUMENT, "NULL argument");
     if (batch < 1 || batch > m->d.maxRows) return fail(ZG_ERR_INVALID_ARGUMENT, "batch must be 1..max_batch");
+    if (mlpFusable(m->d.shape)) { ZG_HIP(mlpFusedTrain(m->d, x, y, (int)batch, lr, s)); return ZG_OK; }
     ZG_HIP(mlpZero(m->d.grad, m->d.nParams, s));
     ZG_HIP(mlpZero(m->d.loss, 1, s));
     ZG_HIP(mlpForward(m->d, x, (int)batch, nullptr, s));
     ZG_HIP(mlpBackward(m->d, y, (int)batch, 1, m->d.loss, nullptr, s));
+    if (lr) { ZG_HIP(mlpAdam(m->d, *lr, s)); }
     return ZG_OK;
 }
 
 zg_status zg_mlp_gradients(zg_mlp* m, const float* x, const float* y, int64_t batch, float* gradHost, float* lossHost,
                            void* stream) {
     hipStream_t s = (hipStream_t)stream;
-    zg_status st = mlpGradientsImpl(m, x, y, batch, s);
+    zg_status st = mlpGradientsImpl(m, x, y, batch, nullptr, s);
     if (st != ZG_OK) return st;
     if (gradHost) { ZG_HIP(hipMemcpyAsync(gradHost, m->d.grad, m->d.nParams * 4, hipMemcpyDeviceToHost, s)); }
     if (lossHost) { ZG_HIP(hipMemcpyAsync(lossHost, m->d.loss, 4, hipMemcpyDeviceToHost, s)); }
@@ -1304,9 +1334,8 @@ zg_status zg_mlp_gradients(zg_mlp* m, const float* x, const float* y, int64_t ba
 zg_status zg_mlp_train_step(zg_mlp* m, const float* x, const float* y, int64_t batch, float lr, float* lossHost,
                             void* stream) {
     hipStream_t s = (hipStream_t)stream;
-    zg_status st = mlpGradientsImpl(m, x, y, batch, s);
+    zg_status st = mlpGradientsImpl(m, x, y, batch, &lr, s);
     if (st != ZG_OK) return st;
-    ZG_HIP(mlpAdam(m->d, lr, s));
     if (lossHost) {
         ZG_HIP(hipMemcpyAsync(lossHost, m->d.loss, 4, hipMemcpyDeviceToHost, s));
         ZG_HIP(hipStreamSynchronize(s));
@@ -1318,6 +1347,12 @@ zg_status zg_mlp_evaluate(zg_mlp* m, const float* x, int64_t n, float* value, fl
     if (!m || (n > 0 && !x)) return fail(ZG_ERR_INVALID_ARGUMENT, "NULL argument");
     hipStream_t s = (hipStream_t)stream;
     int d = m->cfg.in_dim;
+    if (mlpFusable(m->d.shape)) {   // keeps nothing per row: any number of rows, 2^30 at a time
+        for (int64_t r0 = 0; r0 < n; r0 += int64_t(1) << 30)
+            ZG_HIP(mlpFusedEvaluate(m->d, x + r0 * d, (int)std::min<int64_t>(int64_t(1) << 30, n - r0),
+                                    value ? value + r0 : nullptr, gradient ? gradient + r0 * d : nullptr, s));
+        return ok();
+    }
     for (int64_t r0 = 0; r0 < n; r0 += m->d.maxRows) {
         int rows = (int)std::min<int64_t>(m->d.maxRows, n - r0);
         const float* xr = x + r0 * d;

@@ -348,11 +348,13 @@ __global__ void adamKernel(float* __restrict__ theta, float* __restrict__ m, flo
 }
 
 __global__ void castKernel(const float* __restrict__ theta, int64_t n, const int64_t* __restrict__ bfIndex,
-                           uint16_t* __restrict__ bfCopy) {
+                           uint16_t* __restrict__ bfCopy, const int64_t* __restrict__ bfIndexT,
+                           uint16_t* __restrict__ bfT) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     int64_t bi = bfIndex[i];
     if (bi >= 0) bfCopy[bi] = toBf16(theta[i]);
+    if (bi >= 0 && bfT) bfT[bfIndexT[i]] = toBf16(theta[i]);
 }
 
 __global__ void zeroKernel(float* __restrict__ p, int64_t n) {
@@ -383,7 +385,8 @@ hipError_t mlpZero(float* p, int64_t n, hipStream_t s) {
 }
 
 hipError_t mlpCast(MlpDevice& m, hipStream_t s) {
-    hipLaunchKernelGGL(castKernel, dim3(blocks1d(m.nParams)), dim3(256), 0, s, m.theta, m.nParams, m.bfIndex, m.wBf);
+    hipLaunchKernelGGL(castKernel, dim3(blocks1d(m.nParams)), dim3(256), 0, s, m.theta, m.nParams, m.bfIndex, m.wBf,
+                       m.bfIndexT, m.wBfT);
     return hipGetLastError();
 }
 
@@ -426,7 +429,7 @@ hipError_t mlpBackward(MlpDevice& m, const float* y, int n, int mode, float* los
         default: return hipErrorInvalidValue;   // hidden is validated to 1..512
     }
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || mode == 0) return e;   // values only: nothing to propagate
     int cur = 0;
     for (int l = L - 1; l >= 0; l--) {
         int K = l == 0 ? twoF : Hd;
