@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/zombie_amd.h"
 #include "layout.h"
 
@@ -1008,17 +1010,20 @@ struct ExactQuery {
 
 // Complete closest-point query (loops ClosestQuery::visit); see ClosestQuery for the rules.
 // seedPrim >= 0 names a primitive (packed index) likely to be close, tested first.
-template <int D, int W, bool COUNT>
+// EXACT (relax2 = 1, b.obb present): over the oriented boxes, from the seed's entry node.
+template <int D, int W, bool COUNT, bool EXACT = false>
 ZG_DEV bool closestPoint(const BoundaryView& b, const Vec<D>& x, float& best2, Vec<D>& cp, int& prim,
                          Stack& st, VisitCount& vc, float relax2 = 1.0f, float guard2 = 0.0f,
                          float* radius2 = nullptr, int seedPrim = -1) {
-    ClosestQuery<D> q;
+    std::conditional_t<EXACT, ExactQuery<D>, ClosestQuery<D>> q;
     q.begin(best2, relax2, guard2);
     q.cp = cp;
     if (seedPrim >= 0) {
         Prim<D> pr; pr.load(b.prims, seedPrim);
         Vec<D> qq;
-        q.seed(qq, seedPrim, pr.closest2(x, qq));
+        const float s2 = pr.closest2(x, qq);
+        q.seed(qq, seedPrim, s2);
+        if constexpr (EXACT) q.item = entryNode(b.primEntry, seedPrim, s2);
         if (COUNT) vc.prims++;
     }
     st.sp = 0; st.ovf = 0;

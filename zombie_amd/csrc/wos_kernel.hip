@@ -22,7 +22,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
-#include <type_traits>
 
 #include "device.h"
 #include "kernels.h"
@@ -32,7 +31,7 @@ namespace zg {
 // ------------------------------------------------------------------------------------
 // batched queries
 // ------------------------------------------------------------------------------------
-template <int D, int W>
+template <int D, int W, bool EXACT>
 __global__ void __launch_bounds__(256) closestPointKernel(BoundaryView b, int64_t n, const float* __restrict__ pts,
                                                           float* __restrict__ dist, float* __restrict__ closest,
                                                           float* __restrict__ normal, int32_t* __restrict__ prim) {
@@ -44,7 +43,7 @@ __global__ void __launch_bounds__(256) closestPointKernel(BoundaryView b, int64_
     Vec<D> x = vload<D>(pts + i * D);
     float best2 = FLT_MAX;
     Vec<D> cp = vzero<D>(); int pi = -1;
-    bool found = closestPoint<D, W, false>(b, x, best2, cp, pi, st, vc);
+    bool found = closestPoint<D, W, false, EXACT>(b, x, best2, cp, pi, st, vc);
     dist[i] = found ? __builtin_sqrtf(best2) : FLT_MAX;
     if (closest) vstore<D>(closest + i * D, found ? cp : vzero<D>());
     if (normal || prim) {
@@ -757,10 +756,14 @@ hipError_t launchClosestPoint(const SceneView& sv, int boundary, int64_t n, cons
     const BoundaryView& b = boundary ? sv.refl : sv.abs;
     if (n <= 0) return hipSuccess;
     dim3 g(blocksFor(n)), bl(256);
-    if (sv.dim == 2 && sv.width == 4) hipLaunchKernelGGL((closestPointKernel<2, 4>), g, bl, kStackLdsBytes, s, b, n, pts, dist, closest, normal, prim);
-    else if (sv.dim == 2) hipLaunchKernelGGL((closestPointKernel<2, 8>), g, bl, kStackLdsBytes, s, b, n, pts, dist, closest, normal, prim);
-    else if (sv.width == 4) hipLaunchKernelGGL((closestPointKernel<3, 4>), g, bl, kStackLdsBytes, s, b, n, pts, dist, closest, normal, prim);
-    else hipLaunchKernelGGL((closestPointKernel<3, 8>), g, bl, kStackLdsBytes, s, b, n, pts, dist, closest, normal, prim);
+#define ZG_CP(D, Wd)                                                                                                     \
+    do {                                                                                                                 \
+        if (b.obb) hipLaunchKernelGGL((closestPointKernel<D, Wd, true>), g, bl, kStackLdsBytes, s, b, n, pts, dist, closest, normal, prim);  \
+        else hipLaunchKernelGGL((closestPointKernel<D, Wd, false>), g, bl, kStackLdsBytes, s, b, n, pts, dist, closest, normal, prim);       \
+    } while (0)
+    if (sv.dim == 2) { if (sv.width == 4) ZG_CP(2, 4); else ZG_CP(2, 8); }
+    else { if (sv.width == 4) ZG_CP(3, 4); else ZG_CP(3, 8); }
+#undef ZG_CP
     return hipGetLastError();
 }
 
