@@ -145,7 +145,12 @@ __global__ void __launch_bounds__(256) wostGradFirstSphereKernel(WosParams P, fl
 // with an exact absorbing distance and a fresh Green's function (estimateSolution :600-650), and
 // the walk's estimate is the sum over its parts.  When the queue cannot take the copies the walk
 // is not split (an unsplit walk is just as unbiased).
-template <int D, int W, bool COUNT, bool GRAD = false, bool ROBIN = false, bool SPLIT = false>
+// EXACT = true (2D, distance tolerance 0): absorbing distances over the oriented boxes (4,096 segments and 32
+// slits, 10,000 points x 32 walks: 1,000 -> 720 ms).  In 3D the longer query code costs more than the
+// boxes save beside the step's four other traversals (181 VGPRs instead of 155 with 8-wide BVHs; the prism
+// with axis-aligned walls 82-88 ms, 100 ms with oriented boxes, 90 ms with registers capped), so it keeps
+// the axis-aligned ones.
+template <int D, int W, bool EXACT, bool GRAD = false, bool ROBIN = false, bool SPLIT = false>
 __global__ void __launch_bounds__(256) wostKernel(WosParams P) {
     unsigned long long spill[kSpillStack];
     Stack st; st.init(spill);
@@ -247,7 +252,7 @@ __global__ void __launch_bounds__(256) wostKernel(WosParams P) {
         float b2 = FLT_MAX;
         Vec<D> cp = x;
         int prim = -1;
-        bool gotA = closestPoint<D, W, COUNT>(sc.abs, x, b2, cp, prim, st, vc);
+        bool gotA = closestPoint<D, W, false, EXACT>(sc.abs, x, b2, cp, prim, st, vc);
         distA = gotA ? __builtin_sqrtf(b2) : FLT_MAX;
         absPrim = gotA ? prim : -1;
         fsr0 = 0.0f;
@@ -290,7 +295,7 @@ __global__ void __launch_bounds__(256) wostKernel(WosParams P) {
                 int prim = -1;
                 Vec<D> xp = x, nn = nrm;
                 bool al = false;
-                if (closestPoint<D, W, COUNT>(sc.abs, x, b2, cp, prim, st, vc, 1.0f, 0.0f, nullptr, absPrim)) {
+                if (closestPoint<D, W, false, EXACT>(sc.abs, x, b2, cp, prim, st, vc, 1.0f, 0.0f, nullptr, absPrim)) {
                     Prim<D> pr; pr.load(sc.abs.prims, prim);
                     Vec<D> n = pr.normal();
                     float sd = dot(x - cp, n);
@@ -348,7 +353,7 @@ __global__ void __launch_bounds__(256) wostKernel(WosParams P) {
                 float b2 = FLT_MAX;
                 Vec<D> cp = x;
                 int prim = -1;
-                bool gotA = closestPoint<D, W, COUNT>(sc.abs, x, b2, cp, prim, st, vc);
+                bool gotA = closestPoint<D, W, false, EXACT>(sc.abs, x, b2, cp, prim, st, vc);
                 distA = gotA ? __builtin_sqrtf(b2) : FLT_MAX;
                 absPrim = gotA ? prim : -1;
                 nSplits++;
@@ -541,7 +546,7 @@ __global__ void __launch_bounds__(256) wostKernel(WosParams P) {
         // with distance_tolerance > 0 the query returns a certified lower bound of the distance
         // (exact within 2 epsilon of the boundary): a smaller maximal star radius, never a larger one
         float rad2 = FLT_MAX;
-        bool gotA = closestPoint<D, W, COUNT>(sc.abs, x, b2, cp, prim, st, vc, P.relax2, P.guard2, &rad2, absPrim);
+        bool gotA = closestPoint<D, W, false, EXACT>(sc.abs, x, b2, cp, prim, st, vc, P.relax2, P.guard2, &rad2, absPrim);
         distA = gotA ? __builtin_sqrtf(rad2) : FLT_MAX;
         absPrim = gotA ? prim : -1;
         firstStep = false;
@@ -549,10 +554,6 @@ __global__ void __launch_bounds__(256) wostKernel(WosParams P) {
 
     __syncthreads();
     if (threadIdx.x < 6 && blk[threadIdx.x]) atomicAdd(&P.counters[threadIdx.x], blk[threadIdx.x]);
-    if (COUNT) {
-        atomicAdd(&P.counters[kCntNodes], (unsigned long long)vc.nodes);
-        atomicAdd(&P.counters[kCntPrims], (unsigned long long)vc.prims);
-    }
     if (st.overflow) atomicOr(reinterpret_cast<unsigned int*>(&P.counters[kCntError]), 1u);
 }
 
@@ -1207,7 +1208,11 @@ hipError_t launchWostGradFirstSphere(const WosParams& P, int dim, int width, flo
 hipError_t launchWostGrad(const WosParams& P, int dim, int width, int gridBlocks, hipStream_t s) {
     dim3 g(gridBlocks), bl(256);
     const bool robin = !P.pde.are_robin_conditions_pure_neumann;
-#define ZG_WOSTG(Dd, Wd, R) hipLaunchKernelGGL((wostKernel<Dd, Wd, false, true, R>), g, bl, kStackLdsBytes, s, P)
+#define ZG_WOSTG(Dd, Wd, R)                                                                                     \
+    do {                                                                                                      \
+        if (P.exact) hipLaunchKernelGGL((wostKernel<Dd, Wd, Dd == 2, true, R>), g, bl, kStackLdsBytes, s, P);  \
+        else hipLaunchKernelGGL((wostKernel<Dd, Wd, false, true, R>), g, bl, kStackLdsBytes, s, P);         \
+    } while (0)
     if (dim == 3) {
         if (width == 4) { if (robin) ZG_WOSTG(3, 4, true); else ZG_WOSTG(3, 4, false); }
         else { if (robin) ZG_WOSTG(3, 8, true); else ZG_WOSTG(3, 8, false); }
@@ -1241,7 +1246,11 @@ hipError_t launchWost(const WosParams& P, int dim, int width, bool count, bool s
         return hipGetLastError();
     }
     if (split) {   // no visit counting with splitting
-#define ZG_WOSTS(Dd, Wd, R) hipLaunchKernelGGL((wostKernel<Dd, Wd, false, false, R, true>), g, bl, kStackLdsBytes, s, P)
+#define ZG_WOSTS(Dd, Wd, R)                                                                                     \
+    do {                                                                                                      \
+        if (P.exact) hipLaunchKernelGGL((wostKernel<Dd, Wd, Dd == 2, false, R, true>), g, bl, kStackLdsBytes, s, P);  \
+        else hipLaunchKernelGGL((wostKernel<Dd, Wd, false, false, R, true>), g, bl, kStackLdsBytes, s, P);         \
+    } while (0)
         if (dim == 3) {
             if (width == 4) { if (robin) ZG_WOSTS(3, 4, true); else ZG_WOSTS(3, 4, false); }
             else { if (robin) ZG_WOSTS(3, 8, true); else ZG_WOSTS(3, 8, false); }
@@ -1250,7 +1259,11 @@ hipError_t launchWost(const WosParams& P, int dim, int width, bool count, bool s
 #undef ZG_WOSTS
         return hipGetLastError();
     }
-#define ZG_WOST(Dd, Wd, R) hipLaunchKernelGGL((wostKernel<Dd, Wd, false, false, R>), g, bl, kStackLdsBytes, s, P)
+#define ZG_WOST(Dd, Wd, R)                                                                                     \
+    do {                                                                                                      \
+        if (P.exact) hipLaunchKernelGGL((wostKernel<Dd, Wd, Dd == 2, false, R>), g, bl, kStackLdsBytes, s, P);  \
+        else hipLaunchKernelGGL((wostKernel<Dd, Wd, false, false, R>), g, bl, kStackLdsBytes, s, P);         \
+    } while (0)
     if (dim == 3) {
         if (width == 4) { if (robin) ZG_WOST(3, 4, true); else ZG_WOST(3, 4, false); }
         else { if (robin) ZG_WOST(3, 8, true); else ZG_WOST(3, 8, false); }
