@@ -76,8 +76,7 @@ struct DeviceBoundary {
     float* silNodes = nullptr;
     float* silCones = nullptr;
     float silConePrecision = 0.0f;
-    float4* obb = nullptr;       // oriented child boxes (absorbing)
-    float2* primEntry = nullptr; // entry record per packed primitive (absorbing)
+    float4* obb = nullptr;       // oriented child boxes, entry nodes and records (absorbing)
     float* robinMax = nullptr;   // largest Robin coefficient per packed primitive
     BuiltBoundary host;  // sizes only after upload (vectors cleared; reflecting primIds kept)
     int64_t bytes = 0;
@@ -114,7 +113,6 @@ void freeBoundary(DeviceBoundary& b) {
     if (b.silNodes) (void)hipFree(b.silNodes);
     if (b.silCones) (void)hipFree(b.silCones);
     if (b.obb) (void)hipFree(b.obb);
-    if (b.primEntry) (void)hipFree(b.primEntry);
     if (b.robinMax) (void)hipFree(b.robinMax);
     b = DeviceBoundary();
 }
@@ -159,32 +157,33 @@ zg_status buildObb(DeviceBoundary& d, BoundaryView& v) {
     }
     const size_t all = (size_t)n + leafSlots.size() * kEntryLevels;
     if (all > (size_t)INT32_MAX / W) return ZG_OK;
-    const size_t bytes = all * W * ObbLayout<DIM>::kVec * sizeof(float4);
-    float4* obb = nullptr;
-    float2* primEntry = nullptr;
-    int2* dr = nullptr;
-    int32_t* dl = nullptr;
-    hipError_t e = hipMalloc((void**)&obb, bytes);
-    if (e == hipSuccess) e = hipMalloc((void**)&primEntry, (size_t)d.host.nPrims * sizeof(float2));
-    if (e == hipSuccess) e = hipMalloc((void**)&dr, ranges.size() * sizeof(int2));
-    if (e == hipSuccess) e = hipMalloc((void**)&dl, leafSlots.size() * sizeof(int32_t));
+    // one allocation for the boxes and the entry records, one for the build's inputs
+    const size_t boxBytes = all * W * ObbLayout<DIM>::kVec * sizeof(float4), bytes = boxBytes + (size_t)d.host.nPrims * sizeof(float2);
+    const size_t rangeBytes = ranges.size() * sizeof(int2), leafBytes = leafSlots.size() * sizeof(int32_t);
+    std::vector<char> in(rangeBytes + leafBytes);
+    std::memcpy(in.data(), ranges.data(), rangeBytes);
+    std::memcpy(in.data() + rangeBytes, leafSlots.data(), leafBytes);
+    char *out = nullptr, *din = nullptr;
+    hipError_t e = hipMalloc((void**)&out, bytes);
+    if (e == hipSuccess) e = hipMalloc((void**)&din, in.size());
     const bool noRoom = e == hipErrorOutOfMemory;
     if (noRoom) (void)hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpy(dr, ranges.data(), ranges.size() * sizeof(int2), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(dl, leafSlots.data(), leafSlots.size() * sizeof(int32_t), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = launchBuildObb(d.nodes, d.prims, DIM, W, n, dr, obb, 0);
-    if (e == hipSuccess) e = launchBuildEntries(d.nodes, DIM, W, n, dl, (int)leafSlots.size(), obb, primEntry, 0);
+    float4* obb = reinterpret_cast<float4*>(out);
+    float2* primEntry = reinterpret_cast<float2*>(out + boxBytes);
+    if (e == hipSuccess) e = hipMemcpy(din, in.data(), in.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = launchBuildObb(d.nodes, d.prims, DIM, W, n, reinterpret_cast<const int2*>(din), obb, 0);
+    if (e == hipSuccess)
+        e = launchBuildEntries(d.nodes, DIM, W, n, reinterpret_cast<const int32_t*>(din + rangeBytes), (int)leafSlots.size(),
+                               obb, primEntry, 0);
     if (e == hipSuccess) e = hipStreamSynchronize(0);
-    if (dr) (void)hipFree(dr);
-    if (dl) (void)hipFree(dl);
+    if (din) (void)hipFree(din);
     if (e != hipSuccess) {
-        if (obb) (void)hipFree(obb);
-        if (primEntry) (void)hipFree(primEntry);
+        if (out) (void)hipFree(out);
         return noRoom ? ZG_OK : fail(ZG_ERR_DEVICE, "oriented boxes: %s", hipGetErrorString(e));
     }
-    d.obb = obb; d.primEntry = primEntry;
+    d.obb = obb;
     v.obb = obb; v.primEntry = primEntry;
-    d.bytes += (int64_t)(bytes + (size_t)d.host.nPrims * sizeof(float2));
+    d.bytes += (int64_t)bytes;
     return ZG_OK;
 }
 
