@@ -955,15 +955,19 @@ struct ExactQuery {
     bool has;        // an item is held (else pop one)
     bool found;
     bool retried;
+    bool tie;        // with TIES: another primitive is equally near
 
     ZG_DEV void begin(float bound2, float, float) {
+        tie = false;
         best2 = bound2; item = 0; itemD2 = 0.0f; has = true; prim = -1; found = false; retried = false;
     }
     ZG_DEV float radius2() const { return best2; }
     ZG_DEV void seed(const Vec<D>& p, int primIdx, float d2) {
         if (d2 < best2) { best2 = d2; cp = p; prim = primIdx; found = true; }
     }
-    template <int W, bool, class View>
+    // TIES = true keeps track of ties.  Every primitive at the closest distance is tested, since no box bound
+    // exceeds the distances inside it.
+    template <int W, bool, bool TIES = false, class View>
     ZG_DEV bool visit(const View& b, const Vec<D>& x, Stack& st, VisitCount&) {
         if (b.nNodes == 0) return true;
         if (!has) {
@@ -1002,6 +1006,7 @@ struct ExactQuery {
                 Vec<D> qq;
                 const float dd = pr.closest2(x, qq);
                 const bool better = dd < best2;
+                if (TIES) tie = !better && (tie || dd == best2);
 #pragma unroll
                 for (int a = 0; a < D; a++) cp[a] = better ? qq[a] : cp[a];
                 prim = better ? first : prim;
