@@ -47,7 +47,8 @@ __global__ void __launch_bounds__(256) closestPointKernel(BoundaryView b, int64_
     if constexpr (EXACT) {
         // The distance is that of the axis-aligned traversal; which of several equally near primitives (they
         // share the closest vertex or edge) answers is its choice too, so a point with a tie asks it again
-        // (about one point in a hundred; always asking took 10.8 ms where this takes about 1.2 without ties).
+        // (400,000 points of the 81,920-triangle sphere: always asking took 10.7 ms, this takes 3.3, distances alone
+        // about 1.2).
         ExactQuery<D> q;
         q.begin(FLT_MAX, 1.0f, 0.0f);
         q.cp = cp;
