@@ -147,7 +147,7 @@ zg_status buildObb(DeviceBoundary& d, BoundaryView& v) {
         const int32_t* ch = reinterpret_cast<const int32_t*>(nd + L::kChildOffset);
         int lo = INT32_MAX, hi = 0;
         for (int k = 0; k < W; k++) {
-            if (ch[k] == 0) continue;   // empty slot: no child is the root
+            if (L::emptySlot(nd, k)) continue;
             if (ch[k] < 0) leafSlots.push_back(i * W + k);
             const int2 r = ch[k] < 0 ? make_int2(leafFirst(ch[k]), leafCount(ch[k])) : own[ch[k]];
             ranges[(size_t)i * W + k] = r;
@@ -439,6 +439,14 @@ zg_status zg_scene_copy_bvh(const zg_scene* s, int32_t boundary, float* nodes_ho
         return fail(ZG_ERR_INVALID_ARGUMENT, "buffers hold %lld / %lld floats, the BVH needs %lld / %lld",
                     (long long)node_floats, (long long)prim_floats, (long long)nf, (long long)pf);
     if (nodes_host && nf > 0) ZG_HIP(hipMemcpy(nodes_host, b.nodes, (size_t)nf * 4, hipMemcpyDeviceToHost));
+    if (nodes_host) {   // callers know an empty slot by a child of 0
+        const int W = s->width, nodeFloats = (int)(s->info.node_bytes / 4);
+        for (int64_t i = 0; i < b.nNodes; i++) {
+            float* nd = nodes_host + i * nodeFloats;
+            for (int k = 0; k < W; k++)
+                if (NodeLayout<2, 4>::emptySlot(nd, k)) nd[2 * s->dim * W + k] = 0.0f;
+        }
+    }
     if (prims_host && pf > 0) ZG_HIP(hipMemcpy(prims_host, b.prims, (size_t)pf * 4, hipMemcpyDeviceToHost));
     return ok();
 }

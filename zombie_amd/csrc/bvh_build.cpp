@@ -151,7 +151,7 @@ struct WideCollapser {
         float* nd = &out[(size_t)id * L::kFloats];
         for (int k = 0; k < L::kBoxFloats; k++) nd[k] = kEmptyBox;
         int32_t* ch = reinterpret_cast<int32_t*>(nd + L::kChildOffset);
-        for (int k = 0; k < W; k++) ch[k] = 0;
+        for (int k = 0; k < W; k++) ch[k] = kEmptyChild;
         return id;
     }
 

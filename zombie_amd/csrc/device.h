@@ -752,6 +752,17 @@ ZG_DEV void childDistances(const float* nodes, int idx, const Vec<D>& x, float (
     }
 }
 
+// Points that a query can find anything near.  No primitive's distance to any other point compares below a
+// bound, while its NaNs pass the box tests (fmaxf(NaN, 0) is 0, and the projections on an oriented box's axes
+// are NaN once one coordinate is, or two are infinite): the query would visit the whole tree for nothing.
+template <int D>
+ZG_DEV bool isFinite(const Vec<D>& x) {
+    bool ok = true;
+#pragma unroll
+    for (int a = 0; a < D; a++) ok = ok && fabsf(x[a]) <= FLT_MAX;
+    return ok;
+}
+
 // Resumable closest-point query on one boundary part.  A query advances by one work item per
 // call of visit(), so a persistent kernel can interleave the traversals of its lanes with
 // their walk steps instead of making every lane of a wave wait for the slowest traversal.
@@ -791,10 +802,12 @@ struct ClosestQuery {
     bool found;
     bool retried;
 
-    ZG_DEV void begin(float bound2, float relax2_, float guard2_) {
+    // ok = false (a point that is not finite): no item and no second search, nothing is found
+    ZG_DEV void begin(bool ok, float bound2, float relax2_, float guard2_) {
         best2 = bound2; relax2 = relax2_; guard2 = guard2_;
         prune2 = best2 > guard2 ? best2 * relax2 : best2;
-        lower2 = FLT_MAX; item = 0; itemD2 = 0.0f; has = true; prim = -1; found = false; retried = false;
+        has = ok; retried = !ok;
+        lower2 = FLT_MAX; item = 0; itemD2 = 0.0f; prim = -1; found = false;
     }
     ZG_DEV float radius2() const { return fminf(best2, lower2); }
     ZG_DEV void prunedBox(float d2) { if (d2 <= best2) lower2 = fminf(lower2, d2); }
@@ -957,9 +970,10 @@ struct ExactQuery {
     bool retried;
     bool tie;        // with TIES: another primitive is equally near
 
-    ZG_DEV void begin(float bound2, float, float) {
+    ZG_DEV void begin(bool ok, float bound2, float, float) {
         tie = false;
-        best2 = bound2; item = 0; itemD2 = 0.0f; has = true; prim = -1; found = false; retried = false;
+        has = ok; retried = !ok;
+        best2 = bound2; item = 0; itemD2 = 0.0f; prim = -1; found = false;
     }
     ZG_DEV float radius2() const { return best2; }
     ZG_DEV void seed(const Vec<D>& p, int primIdx, float d2) {
@@ -1028,7 +1042,7 @@ ZG_DEV bool closestPoint(const BoundaryView& b, const Vec<D>& x, float& best2, V
                          Stack& st, VisitCount& vc, float relax2 = 1.0f, float guard2 = 0.0f,
                          float* radius2 = nullptr, int seedPrim = -1) {
     std::conditional_t<EXACT, ExactQuery<D>, ClosestQuery<D>> q;
-    q.begin(best2, relax2, guard2);
+    q.begin(isFinite<D>(x), best2, relax2, guard2);
     q.cp = cp;
     if (seedPrim >= 0) {
         Prim<D> pr; pr.load(b.prims, seedPrim);

@@ -5,8 +5,11 @@
 //   float lo[DIM][W]; float hi[DIM][W]; int32 child[W]; padding to NODE_BYTES.
 // child >= 0 : index of an inner node
 // child <  0 : leaf, ~child = (first_prim << 4) | (prim_count - 1)
-// empty slots hold a degenerate box at +1e30 whose squared distance overflows to +inf
-// and whose slab interval lies beyond any ray, so traversal never enters them.
+// empty slots hold a degenerate box at +1e30 whose squared distance overflows to +inf and whose slab
+// interval lies beyond any ray within the scene, so traversal does not enter them.  It would where a
+// comparison says nothing: a NaN coordinate (fmaxf(NaN, 0) is 0), or a ray of unbounded length along a
+// diagonal.  Their code is therefore that of a leaf, the first primitive alone, which is harmless to
+// test; the code of an inner node would lead back into the tree and the traversal would not end.
 //
 // Primitives are stored in leaf order:
 //   3D triangle : 12 floats  a.xyz b.xyz c.xyz, caller index (int bits), 0, 0   (48 B)
@@ -20,6 +23,7 @@
 namespace zg {
 
 constexpr float kEmptyBox = 1e30f;
+constexpr int kEmptyChild = ~0;   // encodeLeaf(0, 1)
 
 template <int DIM, int W>
 struct NodeLayout {
@@ -29,13 +33,14 @@ struct NodeLayout {
     static constexpr int kFloats = ((kRawFloats + 15) / 16) * 16;
     static constexpr int kBytes = kFloats * 4;
     static constexpr int kChildOffset = kBoxFloats;
+    static constexpr __host__ __device__ bool emptySlot(const float* node, int k) { return node[k] >= 0.1f * kEmptyBox; }
 };
 
 // Oriented boxes of the same tree (same node indices, child slots and child codes), read by exact
 // closest-point queries: node n holds its W children one after the other,
 //   3D  64 B: centre.xyz, code; axis0.xyz, half0; axis1.xyz, half1; axis2.xyz, half2
 //   2D  32 B: centre.xy, axis0.xy; half0, half1 (axis1 = axis0 turned by 90 degrees), code, 0
-// An empty slot has half extents of -kEmptyBox: its distance overflows to +inf.
+// An empty slot has half extents of -kEmptyBox: its distance overflows to +inf (its code: kEmptyChild).
 template <int DIM>
 struct ObbLayout {
     static constexpr int kVec = DIM == 3 ? 4 : 2;   // float4 per child

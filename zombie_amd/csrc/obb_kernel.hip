@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(256) buildEntriesKernel(const float* __restric
         const float* nd = nodes + (size_t)node * L::kFloats;
         int keep[W], m = 0;
         for (int k = 0; k < W; k++) {
-            if (__float_as_int(nd[L::kChildOffset + k]) == 0) continue;   // empty slot
+            if (L::emptySlot(nd, k)) continue;
             float d2 = 0.0f;
             for (int a = 0; a < D; a++) {
                 const float g = fmaxf(fmaxf(nd[a * W + k] - hi[a], lo[a] - nd[(D + a) * W + k]), 0.0f);
@@ -220,9 +220,10 @@ __global__ void __launch_bounds__(256) buildEntriesKernel(const float* __restric
     float4* out = obb + (size_t)(nNodes + (int64_t)leaf * kEntryLevels + level) * W * V;
     for (int k = 0; k < W; k++)
         for (int v = 0; v < V; v++) {
-            // an empty slot: half extents of -kEmptyBox
-            float4 e = D == 3 ? make_float4(0.0f, 0.0f, 0.0f, v ? -kEmptyBox : 0.0f)
-                              : (v ? make_float4(-kEmptyBox, -kEmptyBox, 0.0f, 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+            // an empty slot
+            const float none = __int_as_float(kEmptyChild);
+            float4 e = D == 3 ? make_float4(0.0f, 0.0f, 0.0f, v ? -kEmptyBox : none)
+                              : (v ? make_float4(-kEmptyBox, -kEmptyBox, none, 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
             if (k < n) e = obb[(size_t)src[k] * V + v];
             out[k * V + v] = e;
         }

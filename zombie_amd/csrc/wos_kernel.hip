@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(256) closestPointKernel(BoundaryView b, int64_
         // (400,000 points of the 81,920-triangle sphere: always asking took 10.7 ms, this takes 3.3, distances alone
         // about 1.2).
         ExactQuery<D> q;
-        q.begin(FLT_MAX, 1.0f, 0.0f);
+        q.begin(isFinite<D>(x), FLT_MAX, 1.0f, 0.0f);
         q.cp = cp;
         st.sp = 0; st.ovf = 0;
         while (!q.template visit<W, false, true>(b, x, st, vc)) {}
@@ -224,7 +224,7 @@ wosKernel(WosParams P) {
     Vec<D> gB = vzero<D>(), gS = vzero<D>();
     float fsc = 0.0f, cvB = 0.0f, cvS = 0.0f;
     std::conditional_t<EXACT, ExactQuery<D>, ClosestQuery<D>> q;
-    q.begin(FLT_MAX, 1.0f, 0.0f);
+    q.begin(true, FLT_MAX, 1.0f, 0.0f);
     // block counters in LDS: walks per completion code, steps, walks started
     __shared__ unsigned long long blk[6];
     if (threadIdx.x < 6) blk[threadIdx.x] = 0;
@@ -237,11 +237,11 @@ wosKernel(WosParams P) {
             // the algorithmic work of this query: an exact nearest-first traversal of the packed
             // BVH from the root, counted, then discarded (the walk uses its own query below)
             ClosestQuery<D> cq;
-            cq.begin(FLT_MAX, 1.0f, 0.0f);
+            cq.begin(true, FLT_MAX, 1.0f, 0.0f);
             st.sp = 0; st.ovf = 0;
             while (!cq.template visit<W, true>(view, x, st, cvc)) {}
         }
-        q.begin(bound2, relax2, P.guard2);
+        q.begin(true, bound2, relax2, P.guard2);
         q.cp = yc;
         st.sp = 0; st.ovf = 0;
         pendingCode = code;
@@ -501,8 +501,17 @@ wosKernel(WosParams P) {
         if (SCREENED && sigma > 0.0f && ws.steps_before_applying_tikhonov == len) ball.yukawa = true;
         // next radius: the new distance is at most |x - y_prev| (y_prev lies on the boundary)
         float bound2;
-        if (ycValid) bound2 = norm2(x - yc) * 1.0001f + 1e-30f;
-        else { float r2 = 2.0f * R; bound2 = r2 * r2 * 1.0001f + 1e-30f; }
+        if (ycValid) {
+            bound2 = norm2(x - yc) * 1.0001f + 1e-30f;
+        } else {
+            // A walk that has found the boundary moves by that finite distance; one that has not may have
+            // left the finite points, where nothing will be found at any of its steps.  (Its other queries,
+            // one or two a walk, do without the test: beside the walk kernel's spilled registers each
+            // costs the relaxed solve 1%.)
+            if (!isFinite<D>(x)) { dist = FLT_MAX; return; }
+            float r2 = 2.0f * R;
+            bound2 = r2 * r2 * 1.0001f + 1e-30f;
+        }
         beginQuery(bound2, P.relax2, -1);
         if (ycValid && ycPrim >= 0) {
             // the previous closest triangle is usually close to the new closest one: its exact

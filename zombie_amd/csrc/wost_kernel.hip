@@ -707,7 +707,8 @@ __global__ void __launch_bounds__(256) wostInterleavedKernel(WosParams P) {
         qk = kind; stage = kQuery;
         qBest2 = FLT_MAX; qRelax2 = relax2; qGuard2 = guard2;
         qBound = qBest2 > qGuard2 ? qBest2 * qRelax2 : qBest2; qLower2 = FLT_MAX;
-        qItem = 0; qKey = 0.0f; qHas = true; qPrim = -1; qFound = false; qRetried = false;
+        qHas = isFinite<D>(x); qRetried = !qHas;
+        qItem = 0; qKey = 0.0f; qPrim = -1; qFound = false;
         qCp = x;
         st.sp = 0; st.ovf = 0;
         if (absPrim >= 0) {
