@@ -62,6 +62,23 @@ def test_distances_match_brute_force(gpu, kind, width, leaf):
     assert np.abs(d - _brute(V, I, x)).max() <= tol
 
 
+@pytest.mark.parametrize("width,leaf", [(4, 1), (8, 2)])
+def test_boxes_of_a_large_mesh(gpu, width, leaf):
+    """More child slots than the waves that build the boxes take at once (32,768)."""
+    torch = gpu
+    V, I = PB.icosphere(6)
+    V = PB.sh_displace(V, 3).astype(np.float32)
+    I = I.astype(np.int32)
+    x = np.random.default_rng(4).uniform(-1.5, 1.5, (5000, 3)).astype(np.float32)
+    d = []
+    for boundary in (0, 1):
+        sc = E.Scene(V, I, np.full(len(I), boundary, np.uint8), V.min(0) - 1, V.max(0) + 1, bvh_width=width, leaf_size=leaf)
+        nodes = sc.info.n_absorbing_nodes + sc.info.n_reflecting_nodes
+        assert nodes * width > 32768
+        d.append(sc.closest_point(torch.from_numpy(x).cuda(), boundary=boundary, want_point=False)[0])
+    assert torch.equal(*d)
+
+
 @pytest.mark.parametrize("segments,slits", [(64, 1), (700, 6)])
 def test_walk_on_stars_same_walks(gpu, segments, slits):
     torch = gpu

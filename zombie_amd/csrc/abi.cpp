@@ -131,13 +131,14 @@ zg_status uploadBoundary(DeviceBoundary& d, BoundaryView& v) {
     return ZG_OK;
 }
 
-// Adds the oriented child boxes and the entry nodes to an uploaded boundary.  Without memory for them the boundary stays as
-// it is and exact queries use the axis-aligned boxes.
+// Adds the oriented child boxes and the entry nodes to an uploaded boundary.  They are optional: whatever goes
+// wrong (no memory on either side, a launch that is refused), the boundary stays as it is and exact queries
+// use the axis-aligned boxes.  Called last, so that they take no memory that the scene cannot do without.
 template <int DIM, int W>
-zg_status buildObb(DeviceBoundary& d, BoundaryView& v) {
+void buildObb(DeviceBoundary& d, BoundaryView& v) try {
     using L = NodeLayout<DIM, W>;
     const int n = d.host.nNodes;
-    if (n == 0) return ZG_OK;
+    if (n == 0 || n > INT32_MAX / W) return;
     // primitives of every subtree: contiguous, since they are packed in leaf order; children come after
     // their parent
     std::vector<int2> ranges((size_t)n * W, make_int2(0, 0)), own(n);
@@ -156,7 +157,7 @@ zg_status buildObb(DeviceBoundary& d, BoundaryView& v) {
         own[i] = make_int2(lo, hi - lo);
     }
     const size_t all = (size_t)n + leafSlots.size() * kEntryLevels;
-    if (all > (size_t)INT32_MAX / W) return ZG_OK;
+    if (all > (size_t)INT32_MAX / W) return;
     // one allocation for the boxes and the entry records, one for the build's inputs
     const size_t boxBytes = all * W * ObbLayout<DIM>::kVec * sizeof(float4), bytes = boxBytes + (size_t)d.host.nPrims * sizeof(float2);
     const size_t rangeBytes = ranges.size() * sizeof(int2), leafBytes = leafSlots.size() * sizeof(int32_t);
@@ -166,8 +167,6 @@ zg_status buildObb(DeviceBoundary& d, BoundaryView& v) {
     char *out = nullptr, *din = nullptr;
     hipError_t e = hipMalloc((void**)&out, bytes);
     if (e == hipSuccess) e = hipMalloc((void**)&din, in.size());
-    const bool noRoom = e == hipErrorOutOfMemory;
-    if (noRoom) (void)hipGetLastError();
     float4* obb = reinterpret_cast<float4*>(out);
     float2* primEntry = reinterpret_cast<float2*>(out + boxBytes);
     if (e == hipSuccess) e = hipMemcpy(din, in.data(), in.size(), hipMemcpyHostToDevice);
@@ -178,13 +177,14 @@ zg_status buildObb(DeviceBoundary& d, BoundaryView& v) {
     if (e == hipSuccess) e = hipStreamSynchronize(0);
     if (din) (void)hipFree(din);
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         if (out) (void)hipFree(out);
-        return noRoom ? ZG_OK : fail(ZG_ERR_DEVICE, "oriented boxes: %s", hipGetErrorString(e));
+        return;
     }
     d.obb = obb;
     v.obb = obb; v.primEntry = primEntry;
     d.bytes += (int64_t)bytes;
-    return ZG_OK;
+} catch (const std::exception&) {   // the host's memory; nothing is allocated on the device before it
 }
 
 int64_t nodeBytes(int dim, int width) {
@@ -318,11 +318,11 @@ zg_status zg_scene_create(int32_t dim, const float* V, int64_t nV, const int32_t
         return fail(ZG_ERR_INVALID_ARGUMENT, "scene build failed: %s", e.what());
     }
     zg_status st = uploadBoundary(s->abs, s->view.abs);
-    if (st == ZG_OK)
-        st = dim == 2 ? (o.bvh_width == 4 ? buildObb<2, 4>(s->abs, s->view.abs) : buildObb<2, 8>(s->abs, s->view.abs))
-                      : (o.bvh_width == 4 ? buildObb<3, 4>(s->abs, s->view.abs) : buildObb<3, 8>(s->abs, s->view.abs));
     if (st == ZG_OK) st = uploadBoundary(s->refl, s->view.refl);
     if (st != ZG_OK) { freeBoundary(s->abs); freeBoundary(s->refl); delete s; return st; }
+    if (dim == 2) { if (o.bvh_width == 4) buildObb<2, 4>(s->abs, s->view.abs); else buildObb<2, 8>(s->abs, s->view.abs); }
+    else if (o.bvh_width == 4) buildObb<3, 4>(s->abs, s->view.abs);
+    else buildObb<3, 8>(s->abs, s->view.abs);
     s->view.dim = dim; s->view.width = o.bvh_width;
     for (int a = 0; a < 3; a++) {
         s->view.dmin[a] = a < dim && dmin ? dmin[a] : -FLT_MAX;

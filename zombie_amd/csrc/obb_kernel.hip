@@ -1,10 +1,11 @@
 // obb_kernel.hip -- oriented child boxes of a boundary's BVH (layout.h), built once per scene.
 //
-// One wave per child slot reads the child's primitives (a contiguous range) three times: mean normal and
+// One wave at a time reads a child slot's primitives (a contiguous range) three times: mean normal and
 // mean vertex, in-plane covariance, extents.  The frame is the mean normal with the principal in-plane
 // axes; a child whose normals cancel, or whose axis-aligned box is the smaller one, keeps that.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 
 #include "device.h"
@@ -63,14 +64,9 @@ template <int D> ZG_DEV float boxMeasure(const float (&h)[D]) {
     return D == 3 ? h[0] * h[1] + h[1] * h[D - 1] + h[D - 1] * h[0] : h[0] + h[1];
 }
 
+// box of child slot s, whose primitives are [r.x, r.x + r.y), by one wave
 template <int D, int W>
-__global__ void __launch_bounds__(256) buildObbKernel(const float* __restrict__ nodes, const float* __restrict__ prims,
-                                                      int nNodes, const int2* __restrict__ ranges,
-                                                      float4* __restrict__ obb) {
-    const int64_t s = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (s >= (int64_t)nNodes * W) return;
-    const int2 r = ranges[s];
+ZG_DEV void buildBox(const float* nodes, const float* prims, int64_t s, int2 r, int lane, float4* obb) {
     const int code = __float_as_int(nodes[(size_t)(s / W) * NodeLayout<D, W>::kFloats + NodeLayout<D, W>::kChildOffset + s % W]);
     Vec<D> ax[D], c = vzero<D>();
     float half[D];
@@ -138,10 +134,22 @@ __global__ void __launch_bounds__(256) buildObbKernel(const float* __restrict__ 
     }
 }
 
+// A wave takes every (4 gridDim.x)-th slot: with a wave per slot, 2^26 slots (some 60 million triangles in a
+// 4-wide tree) would need more than the 2^32 threads of a launch.
+constexpr int64_t kObbBlocks = 8192;
+
+template <int D, int W>
+__global__ void __launch_bounds__(256) buildObbKernel(const float* __restrict__ nodes, const float* __restrict__ prims,
+                                                      int nNodes, const int2* __restrict__ ranges,
+                                                      float4* __restrict__ obb) {
+    for (int64_t s = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); s < (int64_t)nNodes * W; s += (int64_t)gridDim.x * 4)
+        buildBox<D, W>(nodes, prims, s, ranges[s], threadIdx.x & 63, obb);
+}
+
 hipError_t launchBuildObb(const float* nodes, const float* prims, int dim, int width, int nNodes, const int2* ranges,
                           float4* obb, hipStream_t s) {
     if (nNodes <= 0) return hipSuccess;
-    dim3 g((unsigned)(((int64_t)nNodes * width + 3) / 4)), bl(256);
+    dim3 g((unsigned)std::min(kObbBlocks, ((int64_t)nNodes * width + 3) / 4)), bl(256);
     if (dim == 2 && width == 4) hipLaunchKernelGGL((buildObbKernel<2, 4>), g, bl, 0, s, nodes, prims, nNodes, ranges, obb);
     else if (dim == 2) hipLaunchKernelGGL((buildObbKernel<2, 8>), g, bl, 0, s, nodes, prims, nNodes, ranges, obb);
     else if (width == 4) hipLaunchKernelGGL((buildObbKernel<3, 4>), g, bl, 0, s, nodes, prims, nNodes, ranges, obb);
