@@ -598,6 +598,12 @@ int claimSize(const SolveSetup& S, int64_t walks) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(S.walksPerLane, S.n * walks / (lanes * kClaimsPerLane)));
 }
 
+// Whether boundary data depend on which of several equally near primitives a walk ends at: those that share
+// the closest vertex or edge share the point, but each has a normal of its own.
+bool readsNormal(const zg_function& f) {
+    return f.kind != ZG_FN_DENSE_GRID && (f.eval == ZG_EVAL_NORMAL_DERIVATIVE || f.eval == ZG_EVAL_ROBIN);
+}
+
 // validation and kernel parameters of a walk-on-spheres solve (no allocation, no launch)
 zg_status prepareSolve(const zg_scene* s, const zg_batch* b, const zg_pde* pde, const zg_walk_settings* ws,
                        const zg_sample_points* pts, const int32_t* instanceOf, zg_statistics* stats,
@@ -686,7 +692,15 @@ zg_status prepareSolve(const zg_scene* s, const zg_batch* b, const zg_pde* pde, 
     P.seed = o.seed; P.streamOffset = o.stream_offset;
     P.countMode = o.count_visits;
     P.relax2 = (1.0f - o.distance_tolerance) * (1.0f - o.distance_tolerance);
-    P.exact = o.distance_tolerance == 0.0f && o.count_visits == 0 && (s ? s->view.abs.obb != nullptr : b->hasObb);
+    // Of several equally near primitives the traversals of the two kinds of boxes may name different ones, so
+    // walks whose boundary value reads the primitive's normal keep the axis-aligned boxes, and their value.
+    bool normals = false;
+    if (wost || ws->solve_double_sided) {   // other walks on spheres pass no normal
+        if (s) normals = readsNormal(pde->dirichlet);
+        else for (const zg_pde& ip : b->pdes) normals = normals || readsNormal(ip.dirichlet);
+    }
+    P.exact = o.distance_tolerance == 0.0f && o.count_visits == 0 && !normals &&
+              (s ? s->view.abs.obb != nullptr : b->hasObb);
     float e2 = 2.0f * ws->epsilon_shell_for_absorbing_boundary;
     P.guard2 = e2 * e2 / P.relax2;
 

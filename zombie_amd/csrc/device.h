@@ -957,7 +957,10 @@ ZG_DEV int entryNode(const float2* primEntry, int prim, float s2) {
 // nodes and 143 triangles for the first query of a walk in an 81,920-triangle sphere, 30 and 36 over all
 // queries.  Oriented boxes are as thin as the surface is flat: 21 and 7, 13 and 5.  Walk kernel, issue-bound
 // either way: 100,000 points x 64 walks on that sphere 136 -> 66 ms, 12 screened instances of 2,000 to
-// 200,000 triangles 256 -> 61 ms, 1,024 segments in 2D 15.2 -> 13.5 ms; the same walks, bit for bit.
+// 200,000 triangles 256 -> 61 ms, 1,024 segments in 2D 15.2 -> 13.5 ms.
+//
+// The distance is the same, bit for bit: a minimum over primitives none of which either traversal leaves out
+// wrongly.  Which of several equally near primitives is named depends on the order of the visits.
 template <int D>
 struct ExactQuery {
     Vec<D> cp;       // best point found

@@ -56,7 +56,7 @@ struct WosParams {
     float relax2;        // (1 - distance_tolerance)^2
     float guard2;        // relaxation only when best^2 > guard2 (keeps the shell test exact)
     int32_t nInstances;  // batched solves: size of the instance table
-    int32_t exact;       // distance tolerance 0 and oriented boxes present: queries over the oriented boxes
+    int32_t exact;       // queries over the oriented boxes (distance tolerance 0, boxes present, no tie matters)
     int32_t countMode;   // COUNT kernels: 1 = visits of the kernel's own queries, 2 = visits of an exact
                          // nearest-first traversal from the root at every query point
     double* accSum;
