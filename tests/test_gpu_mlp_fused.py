@@ -43,3 +43,47 @@ def test_fused_shapes_match_oracle(gpu, dim, freq, hidden, layers, rows):
     # the bf16 copies follow the parameters
     cb, _ = M.input_gradient(net.get_parameters(), B, x, hidden, layers, bf16=True)
     assert _rel(net.evaluate(xt, gradient=False)[0].cpu().numpy(), cb) < 2e-3
+
+
+def _near_rounding_boundaries(f, n):
+    """n arguments in [-6, 6] whose f lies within one 32-bit ulp of the middle between two bf16 values."""
+    rng = np.random.default_rng(0)
+    out = np.empty(0, np.float32)
+    while len(out) < n:
+        z = rng.uniform(-6, 6, 1 << 20).astype(np.float32)
+        v = f(z.astype(np.float64))
+        ulp = np.spacing(np.abs(v).astype(np.float32)).astype(np.float64)
+        out = np.concatenate([out, z[np.abs(v / ulp % 65536 - 32768) < 1]])
+    return out[:n]
+
+
+def test_activations_equal_those_of_the_gemm_path(gpu):
+    """The activation and its derivative as the GEMM path computes them (16 and 8 frequencies; an IEEE division
+    each), at pre-activations where half a 32-bit ulp decides the bf16 rounding.  Zero weights make the
+    pre-activations the biases; output weights of +1 and -1 on pairs of equal units make the value exactly 0, so
+    that one row's gradients are the rounded activations (output weights) and derivatives (biases) themselves."""
+    torch = gpu
+    sig = lambda z: 1 / (1 + np.exp(-z))
+    z = np.concatenate([_near_rounding_boundaries(lambda z: z * sig(z), 256),
+                        _near_rounding_boundaries(lambda z: sig(z) * (1 + z * (1 - sig(z))), 256),
+                        # where exp(-z) nears the end of its range and beyond, and where sigmoid is 1
+                        np.linspace(-100, -80, 48), [-1e3, -1e30, -3e38, 0, 1e-30, -1e-30, 16, 17, 18, 80, 100, 1e3, 1e10,
+                                                     1e18, -1e10, -1e18]]).astype(np.float32)
+    x, y = torch.zeros((1, 2), device="cuda"), torch.full((1,), -1.0, device="cuda")
+    got = []
+    for freq in (16, 8):
+        net = LC.MLP(LC.MLPConfig(in_dim=2, n_frequencies=freq, hidden=128, n_hidden_layers=1), max_batch=64)
+        rows = []
+        for zs in z.reshape(-1, 64):
+            theta = np.zeros_like(net.get_parameters())
+            at = 2 * freq * 128
+            theta[at:at + 128] = np.repeat(zs, 2)
+            theta[at + 128:at + 256:2], theta[at + 129:at + 256:2] = 1, -1
+            net.set_parameters(theta)
+            _, g = net.gradients(x, y)
+            rows.append(np.concatenate([g[at:at + 128], g[at + 128:at + 256]]))
+        got.append(np.concatenate(rows))
+    assert np.isfinite(got[0]).all() and (got[0][:8 * 256] != 0).all()
+    # below 2^-126 the reciprocal is 0: activations under 100 * 2^-126 may be too
+    assert ((got[0] == got[1]) | (np.abs(got[0] - got[1]) < 100 * 2.0 ** -126)).all()
+    assert np.array_equal(got[0][:8 * 256], got[1][:8 * 256])
