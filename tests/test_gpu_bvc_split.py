@@ -65,3 +65,42 @@ def test_captured_call(gpu):
         # the chunks' FP64 sums are added in another order
         assert (want.mean - got.mean).abs().max() <= 1e-12 * want.mean.abs().max()
         assert (want.grad_m2 - got.grad_m2).abs().max() <= 1e-10 * want.grad_m2.abs().max()
+
+
+@pytest.mark.parametrize("n", [200, 200000])
+@pytest.mark.parametrize("dim,mu2", [(2, 0.0), (3, 0.0), (3, 2.25)])
+def test_sums_have_no_common_error(gpu, dim, mu2, n):
+    """A pair's estimate e is off by up to ten float roundings, 1e-7 root mean square.  Over many pairs they
+    average out, to 1e-7 sqrt(sum e^2) / |sum e|, which at n = 200,000 is far less than an error that all pairs share,
+    such as that of 1 / (4 pi) rounded to 32 bits (4e-8).  Five standard deviations, and 1e-8 for what is shared."""
+    torch = gpu
+    rng = np.random.default_rng(dim)
+    y = rng.normal(size=(n, dim))
+    y /= np.linalg.norm(y, axis=1, keepdims=True)
+    normal = y.astype(np.float32)
+    y = (y * rng.uniform(0.1, 0.7, (n, 1))).astype(np.float32)
+    f = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.float32)).cuda()
+    one, zero = np.ones(n), np.zeros(n)
+    x = np.zeros((1, dim), np.float32)
+    x[0, 0] = 0.01
+    got, want, tol = [], [], []
+    xy = (x.astype(np.float64) - y)
+    r = np.linalg.norm(xy, axis=1)
+    nx = (xy * normal).sum(1)
+    mr = np.sqrt(mu2) * r
+    G = -np.log(r) / (2 * np.pi) if dim == 2 else np.exp(-mr) / (4 * np.pi * r)
+    K = 1 / (2 * np.pi * r ** 2) if dim == 2 else np.exp(-mr) * (mr + 1) / (4 * np.pi * r ** 3)
+    for src, u in ((True, zero), (False, -one)):   # G alone, P alone (and their squares)
+        s = E.BvcSamples(pt=f(y), normal=f(normal), pdf=f(one), solution=f(u), normal_derivative=f(zero), contribution=f(one),
+                         type=torch.full((n,), A.ZG_SAMPLE_IN_DOMAIN if src else A.ZG_SAMPLE_ON_ABSORBING_BOUNDARY,
+                                         dtype=torch.uint8, device="cuda"))
+        st = E.BvcStats.zeros(1, dim)
+        E.bvc_splat(dim, s, E.BvcEvalPoints(pt=f(x), dist_to_absorbing=f([1.0])), st, absorption=mu2)
+        c = 4 if src else 0
+        e = G if src else nx * K
+        mean, m2 = float(st.mean[0, c]), float(st.m2[0, c])
+        got += [mean, m2 / n + mean ** 2]
+        want += [e.mean(), (e ** 2).mean()]
+        tol += [1e-8 + 5e-7 * np.sqrt((e ** 2).sum()) / abs(e.sum()), 1e-8 + 1e-6 * np.sqrt((e ** 4).sum()) / (e ** 2).sum()]
+    err = np.abs(np.array(got) / want - 1)
+    assert (err <= tol).all(), (err, tol)

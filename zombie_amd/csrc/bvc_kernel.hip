@@ -49,10 +49,19 @@ struct BvcSums {
     double s, q, gs[D], gq[D];
 };
 
+// The loops multiply every estimate by 1 / (4 pi), in 2D 1 / (2 pi), rounded to 32 bits: an error of 4e-8 that all
+// pairs share, where their other roundings average out.  kUnround takes it out of the 64-bit sums.
+constexpr float kInv4Pi = 0.25f / kPi, kLn2 = 0.69314718055994530942f;
+constexpr double kUnround = 0.25 / 3.14159265358979323846 / (double)kInv4Pi;
+
 // Chan merge of a batch into the caller's statistics of point i, category c (common.h:268-310)
 template <int D>
-ZG_DEV void bvcMerge(const zg_bvc_statistics& out, int64_t i, int c, const BvcSums<D>& b) {
+ZG_DEV void bvcMerge(const zg_bvc_statistics& out, int64_t i, int c, BvcSums<D> b) {
     if (b.n == 0) return;
+    b.s *= kUnround;
+    b.q *= kUnround * kUnround;
+#pragma unroll
+    for (int a = 0; a < D; a++) { b.gs[a] *= kUnround; b.gq[a] *= kUnround * kUnround; }
     const size_t k = (size_t)i * kBvcCats + c;
     const int64_t N1 = out.n[k], nb = b.n, N = N1 + nb;
     const double f2 = (double)nb / (double)N, f12 = (double)N1 * (double)nb / (double)N;
@@ -185,11 +194,14 @@ __global__ void __launch_bounds__(64) bvcSplatKernel(BvcParams B) {
                 // grad P = [n - (x - y) 2 n.(x - y) / r^2] / (2 pi r^2)
                 float G, K, Q;   // grad G = -(x - y) K, P = n.(x - y) K, grad P = n K - (x - y) Q
                 if constexpr (D == 2) {
-                    G = logf(r2) * (-0.25f / kPi);
-                    K = inv2 * (0.5f / kPi);
+                    // v_log_f32 rounds down, which over many pairs is a common error of half an ulp (4e-8), in logf
+                    // too; that of -log(1 / r2) is the opposite
+                    const float l2 = __builtin_amdgcn_logf(inv2) - __builtin_amdgcn_logf(r2);
+                    G = l2 * (0.5f * kLn2) * kInv4Pi;
+                    K = inv2 * (2.0f * kInv4Pi);
                     Q = 2.0f * (nx * inv2) * K;
                 } else {
-                    const float g0 = inv * (0.25f / kPi), g2 = inv2 * g0;
+                    const float g0 = inv * kInv4Pi, g2 = inv2 * g0;
                     if constexpr (YUKAWA) {
                         const float mr = B.mu * (r2 * inv), e = expf(-mr);
                         G = e * g0;
