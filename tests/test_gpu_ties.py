@@ -6,6 +6,7 @@ import pytest
 
 from zombie_amd import _abi as A
 from zombie_amd import engine as E
+from zombie_amd import problems as PB
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +43,42 @@ def test_boundary_data_that_read_the_normal(gpu, kind, double_sided, eval_):
         out.append(st)
     assert torch.equal(out[0].walk_length, out[1].walk_length)
     assert (out[0].mean - out[1].mean).abs().max() <= walks * 2.0 ** -52
+
+
+def _mesh(dim):
+    """Nonconvex shapes whose vertices (and edges) are closest for whole regions of points, inside and outside."""
+    if dim == 2:
+        return _gear()
+    V, I = PB.icosphere(2)
+    V = V * (1.0 + 0.3 * np.sin(5 * V[:, :1]) * np.cos(7 * V[:, 1:2]))
+    return V.astype(np.float32), I.astype(np.int32)
+
+
+@pytest.mark.parametrize("dim,width,leaf", [(2, 4, 2), (2, 8, 4), (3, 4, 1), (3, 4, 2), (3, 8, 4)])
+def test_closest_point_names_the_same_primitive(gpu, dim, width, leaf):
+    """Point, normal and primitive of every query equal those of the axis-aligned traversal (the same mesh as a
+    reflecting boundary), bit for bit: in the regions of vertices and edges, on them, and anywhere."""
+    torch = gpu
+    V, I = _mesh(dim)
+    rng = np.random.default_rng(5)
+    T = V[I].astype(np.float64)
+    edges = np.concatenate([T[:, [a, (a + 1) % dim]] for a in range(dim)])
+    mid = edges[rng.integers(0, len(edges), 4000)]
+    w = rng.random((4000, 1))
+    on_edge = mid[:, 0] * w + mid[:, 1] * (1 - w)
+    x = np.concatenate([V, V * 1.3, V * 0.8, on_edge, on_edge * 1.2, on_edge * 0.9,
+                        rng.uniform(-1.6, 1.6, (8000, dim))]).astype(np.float32)
+    out = []
+    for boundary in (0, 1):
+        sc = E.Scene(V, I, np.full(len(I), boundary, np.uint8), V.min(0) - 1, V.max(0) + 1, bvh_width=width, leaf_size=leaf)
+        r = sc.closest_point(torch.from_numpy(x).cuda(), boundary=boundary, want_normal=True, want_prim=True)
+        out.append([a.cpu().numpy() for a in r])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    # ties take part: the brute-force minimum is shared by several primitives for many of these points
+    d, _, _, prim = out[0]
+    a, e = T[:, 0], T[:, 1] - T[:, 0]
+    if dim == 2:
+        t = np.clip(((x[:, None] - a) * e).sum(-1) / (e * e).sum(-1), 0, 1)
+        all_d = np.linalg.norm(x[:, None] - a - t[..., None] * e, axis=-1)
+        assert ((all_d <= all_d.min(1, keepdims=True) + 1e-7).sum(1) > 1).mean() > 0.2
