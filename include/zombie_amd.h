@@ -164,7 +164,10 @@ typedef struct zg_scene_info {
  * and populateGeometricQueriesFor{Dirichlet,Neumann}Boundary (:1062-1304); for the
  * reflecting part the silhouette candidates of computeSilhouettes (:631, :667) -- vertices in
  * 2D, edges in 3D -- are built with getIgnoreCandidateSilhouetteCallback(solve_double_sided,
- * silhouette_precision) (:1029-1038; 3D dihedral angle as :955-967 measures it). */
+ * silhouette_precision) (:1029-1038; 3D dihedral angle as :955-967 measures it).
+ * The absorbing part also gets oriented boxes, which exact queries and walks read (device_bytes
+ * counts them: about 25 MB beside 5 MB for 81,920 triangles); a scene is created without them
+ * where they cannot be had, and answers the same more slowly. */
 zg_status zg_scene_create(int32_t dim, const float* positions_host, int64_t n_vertices,
                           const int32_t* indices_host, int64_t n_prims,
                           const uint8_t* is_reflecting_host,
@@ -506,8 +509,11 @@ typedef struct zg_bvc_statistics {
  * derivative of P, where the reference's formula at :307-317 differs) -- optional kernel regularization
  * (distributions.h:12-55), the Robin / Neumann / Dirichlet forms of the boundary estimate,
  * alpha = 2 for evaluation points on the boundary (gradient 0 there); evaluation points closer
- * than the cutoffs to the boundaries are skipped; non-finite kernels skip the sample.  One
- * thread per evaluation point, samples staged through LDS.  absorption >= 0; > 0 in 2D is
+ * than the cutoffs to the boundaries are skipped; non-finite kernels skip the sample.  A wave
+ * per 64 evaluation points and chunk of the samples; where several chunks are needed to fill
+ * the GPU, their sums go through a workspace (at most 140 MB) taken from the stream's memory pool
+ * (hipMallocAsync) and given back on the stream by every call.  A call that is being captured, or
+ * finds no memory, takes one chunk and no workspace.  absorption >= 0; > 0 in 2D is
  * ZG_ERR_UNSUPPORTED (screened Poisson runs in 3D). */
 zg_status zg_bvc_splat(int32_t dim, float absorption, const zg_bvc_samples* samples_host,
                        const zg_bvc_eval_points* eval_host, float radius_clamp, float kernel_regularization,

@@ -1020,8 +1020,10 @@ zg_status zg_bvc_splat(int32_t dim, float absorption, const zg_bvc_samples* S, c
     if (!(radiusClamp >= 0.0f) || !(kreg >= 0.0f)) return fail(ZG_ERR_INVALID_ARGUMENT, "radius clamp and kernel regularization must be >= 0");
     int dev = 0;
     ZG_HIP(hipGetDevice(&dev));
-    // 12 waves per CU: what the splat's 145 registers allow in 3D (16 / 32 / 64 ran 1.77 / 1.64 / 1.69 ms where
-    // 12 took 1.50)
+    // 12 waves per CU: three per SIMD, what the splat's registers allow in 3D.  10,000 points x (40,000 + 10,000
+    // samples), alone and among other calls: 8 / 12 / 16 / 32 ran 1.16 / 1.42 / 1.67 / 1.56 and 1.03 / 1.03 /
+    // 1.02 / 0.94 ms in 3D, 1.11 / 0.96 / 1.29 / 1.46 and 1.03 / 0.87 / 0.89 / 0.84 in 2D.  None is best throughout;
+    // 12 is within 10% of the best in three of the four, on two fifths of the workspace of 32
     hipError_t e = launchBvcSplat(dim, absorption, *S, *E, *out, radiusClamp, kreg, robinCutoff, cutoffA, cutoffR,
                                   12 * cuCount(dev), (hipStream_t)stream);
     if (e != hipSuccess) return fail(ZG_ERR_DEVICE, "zg_bvc_splat: %s", hipGetErrorString(e));

@@ -14,8 +14,8 @@
 // Bound: VALU issue (about 50 FP32 and 12 FP64 instructions per pair in 3D).  Splitting the samples
 // over blockIdx.y keeps the chip full when the evaluation points alone are too few waves; the chunks'
 // sums then go through a workspace that a second kernel adds up in order.  10,000 points x (40,000
-// boundary + 10,000 source samples) in 3D: 38.5 ms with one 256-thread block per 256 points and the
-// divisions in the loop, 1.5 ms now (2D: 32.8, 1.1).
+// boundary + 10,000 source samples) in 3D, both splats: 38.5 ms with one 256-thread block per 256 points and
+// the divisions in the loop, 1.0 ms now among other calls and 1.4 alone (2D: 32.8, 0.9 and 1.0).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

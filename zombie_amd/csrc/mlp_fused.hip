@@ -10,12 +10,12 @@
 // activations and their gradients), which one more kernel contracts, and a third adds up the partial
 // gradients and takes the Adam step.
 //
-// Measured at 128 units, 4 layers, 64 features: a training step of 65,536 rows 350 -> 94 us (fused layers 61,
-// weight gradients 24, reduction and Adam 9), 262,144 values and gradients 1,010 -> 230 us.  Bound: the chain
-// of barriers and dependent products within a tile (VALU issue, mostly the activations, is a third of the
-// time).  What it took: weights stored in the order of the MFMA operand (a row-major load touches 32 cache
-// lines), 16 waves of 16 x 32 results instead of 8 of 32 x 32 (95 -> 71 us once nothing spilled), and no
-// 64-bit address or old pre-activation held per lane (spills: 121 -> 71 -> 61 us).
+// Measured at 128 units, 4 layers, 64 features: a training step of 65,536 rows 350 -> 96 us of kernels (fused
+// layers 63, weight gradients 24, reduction and Adam 9), 262,144 values and gradients 1,010 -> 205 us.  Bound: the
+// chain of barriers and dependent products within a tile (VALU issue, mostly the activations, is a third of
+// the time).  What it took: weights stored in the order of the MFMA operand (a row-major load touches 32
+// cache lines), 16 waves of 16 x 32 results instead of 8 of 32 x 32 (95 -> 71 us once nothing spilled), and no
+// 64-bit address or old pre-activation held per lane (spills: 121 -> 71 -> 61 us, before the divisions below).
 //
 // Precision is that of the GEMM per layer: bf16 operands, 32-bit products, sums, pre-activations and
 // derivatives, divisions as an IEEE division rounds them; the sums are taken in another order.
@@ -341,7 +341,8 @@ __global__ void __launch_bounds__(8 * H) fusedKernel(FusedArgs g) {
 // sums of their own.  MFMA v_mfma_f32_32x32x16_bf16, lane l of 64 (half = l / 32), element j of 8 / e of 16:
 //   A[row = l % 32][k = 8 half + j],  B[k = 8 half + j][col = l % 32],
 //   D[row = 8 (e / 4) + 4 half + e % 4][col = l % 32]
-// Reads both operands once past L2 (134 MB at a batch of 65,536).
+// Reads both operands once past L2 (126 MB at a batch of 65,536 with 4 layers: 4 gradients and 3 activations of
+// 16.8 MB, 8.4 MB of features).
 struct WeightArgs {
     int rowBlocks, F, L, splits;
     const uint16_t* phiBlk;
@@ -456,6 +457,9 @@ __global__ void __launch_bounds__(256) reduceKernel(ReduceArgs g, int weightBloc
 // ------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------
+// More units, features or layers do not fit a block's registers and LDS.  The smaller shapes between (32 or 96
+// units, 8 or 24 frequencies) would, but are not among the kernel's instances: they take a GEMM per layer, 230
+// to 330 us per training step of 65,536 rows with 4 layers where the fused shapes around them take 59 to 100.
 bool mlpFusable(const MlpShape& s) {
     return (s.hidden == 64 || s.hidden == 128) && (s.nFreq == 16 || s.nFreq == 32) && s.nHidden <= kFusedLayers;
 }

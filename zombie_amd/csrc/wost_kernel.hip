@@ -146,10 +146,12 @@ __global__ void __launch_bounds__(256) wostGradFirstSphereKernel(WosParams P, fl
 // the walk's estimate is the sum over its parts.  When the queue cannot take the copies the walk
 // is not split (an unsplit walk is just as unbiased).
 // EXACT = true (2D, distance tolerance 0): absorbing distances over the oriented boxes (4,096 segments and 32
-// slits, 10,000 points x 32 walks: 1,000 -> 720 ms).  In 3D the longer query code costs more than the
-// boxes save beside the step's four other traversals (181 VGPRs instead of 155 with 8-wide BVHs; the prism
-// with axis-aligned walls 82-88 ms, 100 ms with oriented boxes, 90 ms with registers capped), so it keeps
-// the axis-aligned ones.
+// slits, 10,000 points x 32 walks: 1,066 -> 776 ms).  3D keeps the axis-aligned ones, because the longer query
+// code costs registers (181 VGPRs instead of 155 with 8-wide BVHs) that flat walls along the axes do not pay back:
+// 20,000 points x 64 walks in the prism 83 ms, 98 with oriented boxes (90 with registers capped).  It is
+// the slower choice where the absorbing surface is curved: in displaced spheres of 5,120 / 81,920 triangles,
+// a quarter of them Neumann, 83 / 262 ms against 56 / 98 with 8-wide BVHs, 67 / 234 against 36 / 64 with 4-wide ones.
+// A choice per scene is not made.
 template <int D, int W, bool EXACT, bool GRAD = false, bool ROBIN = false, bool SPLIT = false>
 __global__ void __launch_bounds__(256) wostKernel(WosParams P) {
     unsigned long long spill[kSpillStack];
