@@ -116,3 +116,15 @@ def test_walks_on_stars_from_such_points_end(gpu, dim, interleave):
     st = E.DeviceStats.zeros(n)
     E.wost_solve(sc, p.pde, ws, dp, st, E.SolveOptions(seed=5, wost_interleave_queries=interleave))
     assert torch.isfinite(st.mean[torch.from_numpy(ordinary).cuda()]).all()
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("width", [4, 8])
+def test_copied_tree_has_zeros_in_empty_slots(gpu, dim, width):
+    V, I = _mesh(dim)
+    sc = E.Scene(V, I, None, V.min(0) - 1, V.max(0) + 1, bvh_width=width, leaf_size=1)
+    nodes, _ = sc.copy_bvh(0)
+    nodes = nodes.reshape(sc.info.n_absorbing_nodes, -1)
+    child = nodes.view(np.int32)[:, 2 * dim * width:(2 * dim + 1) * width]
+    empty = nodes[:, :width] == np.float32(1e30)
+    assert empty.any() and np.array_equal(child == 0, empty)
